@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "dugma_internal.h"
+#include "dugma_near.h"
 #include "dugma_pairs.h"
 
 namespace dugma {
@@ -265,6 +266,7 @@ static void free_ctx(dugma_ctx *c) {
                   c->dSrecF, c->dSrecI};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
+  c->nearbuf.release();
   c->part.release();
   c->scratch2.release();
   c->sigbuf.release();
@@ -333,7 +335,7 @@ extern "C" int dugma_init(const double *X, const double *X_C, const double *Y,
     e = hipHostGetDevicePointer((void **)&c->dres, c->hres, 0);
     if (e != hipSuccess) TRY(hip_fail(e, "hipHostGetDevicePointer"));
     e = hipHostMalloc((void **)&c->hparts, sizeof(double) * kPosePart * dugma_ctx::kHostParts,
-                      hipHostMallocDefault);
+                      hipHostMallocCoherent);
     if (e != hipSuccess) {
       c->hparts = nullptr;
       TRY(hip_fail(e, "hipHostMalloc(parts)"));
@@ -383,13 +385,22 @@ extern "C" int dugma_init(const double *X, const double *X_C, const double *Y,
     bool isoT = true, isoS = true;
     double logv = 0.0;
     long nlog = 0;
-    auto consider = [&](const double *P, const double *C, int n, std::vector<int> &keep, bool &iso) {
+    double lo[2][3], hi[2][3];  // bounds of the kept points
+    auto consider = [&](const double *P, const double *C, int n, std::vector<int> &keep, bool &iso, int w) {
+      for (int a = 0; a < 3; ++a) {
+        lo[w][a] = INFINITY;
+        hi[w][a] = -INFINITY;
+      }
       double p32[3], c32[9];
       for (int i = 0; i < n; ++i) {
         for (int a = 0; a < D; ++a) p32[a] = f32(P[(size_t)i * D + a]);
         for (int a = 0; a < DD; ++a) c32[a] = f32(C[(size_t)i * DD + a]);
         if (!valid_point(D, p32, c32)) continue;
         keep.push_back(i);
+        for (int a = 0; a < D; ++a) {
+          lo[w][a] = std::min(lo[w][a], p32[a]);
+          hi[w][a] = std::max(hi[w][a], p32[a]);
+        }
         iso = iso && isotropic(D, c32);
         double tr = 0;
         for (int a = 0; a < D; ++a) tr += c32[a * (D + 1)];
@@ -397,8 +408,8 @@ extern "C" int dugma_init(const double *X, const double *X_C, const double *Y,
         ++nlog;
       }
     };
-    consider(X, X_C, N, keepT, isoT);
-    consider(Y, Y_C, M, keepS, isoS);
+    consider(X, X_C, N, keepT, isoT, 0);
+    consider(Y, Y_C, M, keepS, isoS, 1);
     c->nT = (int)keepT.size();
     c->nS = (int)keepS.size();
     c->isoT = isoT;
@@ -446,6 +457,7 @@ extern "C" int dugma_init(const double *X, const double *X_C, const double *Y,
       if (e3 == hipSuccess) e3 = hipMemcpy(c->dSsrc, src.data(), sizeof(double) * src.size(), hipMemcpyHostToDevice);
     }
     if (e3 != hipSuccess) TRY(hip_fail(e3, "dugma_init: energy-state upload"));
+    TRY(near_build(c, lo, hi));
     c->hTidx = std::move(keepT);
     c->hSidx = std::move(keepS);
     c->hSsrc = std::move(src);

@@ -1,18 +1,14 @@
 // dugma_energy.hip -- convolved-uncertainty energy, fused pose adjoint,
 // per-point adjoint and the finite-difference ("plain") gradient.
 //
-// Kernel shape: a workgroup is 4 waves; each lane owns T stationary points
-// in VGPRs (the transformed sources in the pose and energy passes; targets,
-// then sources, in the two per-point passes) and walks a chunk of the other
-// cloud.  The streamed records are read with wave-uniform
-// addresses, so they come through the scalar cache into SGPRs and feed the
-// VALU directly: no LDS, no barriers in the pair loop.  (On gfx950 an
-// instruction with an SGPR operand issues at about half the rate of an
-// all-VGPR one, but staging the records in LDS and reading them into VGPRs
-// was slower: the wave-wide LDS reads become the bound.)  Per-pair terms are
-// FP32, summed in FP32 over sub-tiles of kSub streamed points and then in
-// FP64 per lane; workgroup partials are reduced in a fixed order, so results
-// are deterministic run to run.  Nothing of size N x M is stored.
+// Kernel shape (k_near): a workgroup takes 64 stationary points, one per lane
+// of each of its 8 waves (the transformed sources in the pose and energy passes;
+// targets, then sources, in the two per-point passes), finds the points of the
+// other cloud that any of them can have a term other than exactly 0 with, and
+// sums those pairs.  Per-pair terms are FP32, summed in FP32 over sub-tiles of
+// kSub streamed points in their own order and then in FP64 per lane;
+// workgroup partials are reduced in a fixed order, so results are
+// deterministic run to run.  Nothing of size N x M is stored.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -23,18 +19,19 @@
 #include <vector>
 
 #include "dugma_internal.h"
+#include "dugma_near.h"
 #include "dugma_pairs.h"
 
 namespace dugma {
 
 constexpr int kBlock = 256;  // 4 waves of 64
 constexpr int kSub = 64;     // FP32 sub-tile length before the FP64 flush
-constexpr int kMinChunk = 32;  // fewest streamed points per workgroup
+constexpr int kMinChunk = 32;  // fewest streamed points per chunk
 
 // kModeHess: the pose pass plus the sums of an approximate pose Hessian
 // (3-D, transformed sources stationary)
 enum { kModeEnergy = 0, kModePose = 1, kModePoint = 2, kModeHess = 3 };
-constexpr int kHessPart = 32;  // per workgroup: the kPosePart pose values, then 21 Hessian entries
+constexpr int kHessPart = 32;  // doubles per workgroup of k_hess_tiles (21 used)
 
 __device__ __forceinline__ float wave_sum_f(float v) {
 #pragma unroll
@@ -76,25 +73,144 @@ struct PoseArg {
 };
 
 // ---------------------------------------------------------------------------
+// Per-call source records: x' = R x + t and S' = R S R^T in FP64, then
+// split to FP32 hi/lo (positions) and rounded (covariance).
+// ---------------------------------------------------------------------------
+template <int D>
+__device__ __forceinline__ void transform_pos(const double *__restrict__ s, const PoseArg &ps, float *hi, float *lo) {
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    double v = ps.t[a];
+#pragma unroll
+    for (int b = 0; b < D; ++b) v = fma(ps.R[a + D * b], s[b], v);
+    hi[a] = (float)v;
+    lo[a] = (float)(v - (double)hi[a]);
+  }
+}
+// S' = R S R^T (column-major)
+template <int D>
+__device__ __forceinline__ void transform_cov(const double *__restrict__ S, const PoseArg &ps, double *Sp) {
+  double RS[9];
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      double v = 0.0;
+#pragma unroll
+      for (int b = 0; b < D; ++b) v = fma(ps.R[a + D * b], S[b + D * c], v);
+      RS[a + D * c] = v;
+    }
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      double v = 0.0;
+#pragma unroll
+      for (int b = 0; b < D; ++b) v = fma(RS[a + D * b], ps.R[c + D * b], v);
+      Sp[a + D * c] = v;
+    }
+}
+__device__ __forceinline__ void transform_rec(const double *__restrict__ s, const PoseArg &ps, Rec3I &r) {
+  float hi[3], lo[3];
+  transform_pos<3>(s, ps, hi, lo);
+  r.hx = hi[0]; r.hy = hi[1]; r.hz = hi[2];
+  r.lx = lo[0]; r.ly = lo[1]; r.lz = lo[2];
+  r.s = (float)(s[3] * kLn4);
+  r.pad0 = 0.0f;
+}
+__device__ __forceinline__ void transform_rec(const double *__restrict__ s, const PoseArg &ps, Rec2I &r) {
+  float hi[3], lo[3];
+  transform_pos<2>(s, ps, hi, lo);
+  r.hx = hi[0]; r.hy = hi[1]; r.lx = lo[0]; r.ly = lo[1];
+  r.s = (float)(s[2] * kLn4);
+  r.pad0 = r.pad1 = r.pad2 = 0.0f;
+}
+__device__ __forceinline__ void transform_rec(const double *__restrict__ s, const PoseArg &ps, Rec3F &r) {
+  float hi[3], lo[3];
+  double Sp[9];
+  transform_pos<3>(s, ps, hi, lo);
+  transform_cov<3>(s + 3, ps, Sp);
+  r.hx = hi[0]; r.hy = hi[1]; r.hz = hi[2];
+  r.lx = lo[0]; r.ly = lo[1]; r.lz = lo[2];
+  r.s11 = (float)Sp[0];
+  r.s22 = (float)Sp[4];
+  r.s33 = (float)Sp[8];
+  r.s12 = (float)(0.5 * (Sp[3] + Sp[1]));
+  r.s13 = (float)(0.5 * (Sp[6] + Sp[2]));
+  r.s23 = (float)(0.5 * (Sp[7] + Sp[5]));
+  r.pad0 = r.pad1 = r.pad2 = r.pad3 = 0.0f;
+}
+__device__ __forceinline__ void transform_rec(const double *__restrict__ s, const PoseArg &ps, Rec2F &r) {
+  float hi[3], lo[3];
+  double Sp[9];
+  transform_pos<2>(s, ps, hi, lo);
+  transform_cov<2>(s + 2, ps, Sp);
+  r.hx = hi[0]; r.hy = hi[1]; r.lx = lo[0]; r.ly = lo[1];
+  r.s11 = (float)Sp[0];
+  r.s22 = (float)Sp[3];
+  r.s12 = (float)(0.5 * (Sp[2] + Sp[1]));
+  r.pad0 = 0.0f;
+}
+
+template <class Rec>
+__global__ __launch_bounds__(kBlock) void k_transform_src(
+    const double *__restrict__ src, int n, PoseArg ps, Rec *__restrict__ out) {
+  constexpr int D = RecTraits<Rec>::D;
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= n) return;
+  Rec r;
+  transform_rec(src + (size_t)k * (D + D * D), ps, r);
+  out[k] = r;
+}
+
+// ---------------------------------------------------------------------------
 // Pair kernel
 // ---------------------------------------------------------------------------
-// With one stationary point per lane every variant fits in 64 VGPRs (no
-// scratch), which allows 8 waves per SIMD instead of 6; two per lane need
-// more registers and keep the compiler's default.
+// One workgroup (8 waves) takes 64 stationary points that are neighbours in
+// Hilbert order, one per lane of every wave, and the part qc of qsplit of the
+// streamed cloud's sub-tiles (groups of up to kSub consecutive points, the FP32
+// sums' unit).
 //
-// Tiles are (stationary block, streamed chunk) pairs.  With xcd_map set
-// they lie on a 1-D grid mapped XCD-aware: workgroups are dispatched to the 8
-// XCDs round-robin, so XCD x runs workgroups x, x + 8, ...; each XCD takes a
-// contiguous eighth of the stationary blocks (bpx of them) and walks every
-// streamed chunk across them, chunk by chunk.  A chunk is then fetched into
-// an XCD's L2 once and used by its bpx blocks, and the XCD's stationary
-// records (an eighth of them) stay in that L2 for every chunk.  The grid is
-// padded to 8 x bpx x qchunks workgroups; the padding exits at once.
-// Without xcd_map (clouds that fit one L2 anyway) the grid is 2-D:
-// block blockIdx.x of chunk blockIdx.y.
+// 1. Wave 0 reads the stationary points (XSRC: transforms them from the FP64
+//    source data, so that no launch has to do it first) and leaves them and
+//    the boxes of their 4 rows of 16 and 16 quads of 4 in LDS.
+// 2. The lanes test the streamed cloud's 64-point boxes against the rows, then
+//    the points of the boxes that are near against rows and quads, and set a
+//    bit in LDS for each point that any of the 64 lanes may have a term other
+//    than 0 with.  Bits stand in the streamed points' own order, group by
+//    group.
+// 3. Each wave turns its groups' set bits into a list (LDS), takes 16 entries
+//    at a time -- lane l loads the record of entry l % 16, so every row of 16
+//    lanes holds the 16 records -- and adds their pairs one after another, the
+//    record's words broadcast within the rows by the consuming instruction
+//    (DPP row_newbcast, which issues at the rate of an SGPR operand).  Points
+//    without a bit add exactly 0 for every lane, so the FP32 sums of a group are
+//    those of all its points, in their order.
+//
+// What bounds it: at 200K x 200K (isotropic, 8-NN sigma) a workgroup lists 3,200
+// of 200,000 streamed points, 1,450 of which any one lane needs; FP32 issue of
+// those pairs and the FP64 flush of their 2,000 sub-tiles.  0.79 ms against
+// 18.4 ms with every pair evaluated (outputs equal to 2e-16).  6,000 x 6,000
+// full covariances: 24 us against 66 (160 listed of 6,000; a chain of
+// dependent loads).  Scalar loads of the listed records (each wave at its own
+// addresses) were bound by the scalar cache's misses, 145 cycles per record
+// and CU: 1.86 ms at 200K.
+constexpr int kCap = 256;  // list entries per wave (whole groups at a time)
+constexpr int kNearBlock = 512;
+constexpr int kNearWaves = kNearBlock / 64;
+constexpr int kRows = 4, kQuads = 16;  // boxes of 16 and of 4 stationary points
+// LDS for the bits: 2^18 points (32 KiB); larger clouds go window by window.
+constexpr int kWinGroups = 4096;
+
+// Tiles are (stationary block, part) pairs.  With xcd_map set they lie on a
+// 1-D grid mapped XCD-aware: workgroups are dispatched to the 8 XCDs
+// round-robin, so XCD x runs workgroups x, x + 8, ...; each XCD takes a
+// contiguous eighth of the stationary blocks, whose near streamed points are
+// about an eighth of that cloud and stay in its L2.
+// Without xcd_map (clouds that fit one L2 anyway) the grid is 2-D.
 constexpr int kXcds = 8;
 constexpr size_t kXcdMapBytes = size_t(4) << 20;  // both clouds' records beyond one XCD's L2 (4 MiB)
-__device__ __forceinline__ bool xcd_tile(int pblocks, int qchunks, int xcd_map, int *sb, int *qc) {
+__device__ __forceinline__ bool xcd_tile(int pblocks, int qsplit, int xcd_map, int *sb, int *qc) {
   if (!xcd_map) {
     *sb = blockIdx.x;
     *qc = blockIdx.y;
@@ -105,63 +221,351 @@ __device__ __forceinline__ bool xcd_tile(int pblocks, int qchunks, int xcd_map, 
   const int xcd = g % kXcds, local = g / kXcds;
   *sb = xcd * bpx + local % bpx;
   *qc = local / bpx;
-  return *sb < pblocks && *qc < qchunks;
+  return *sb < pblocks && *qc < qsplit;
 }
-static inline dim3 tile_grid(int pblocks, int qchunks, int xcd_map) {
-  return xcd_map ? dim3(kXcds * ((pblocks + kXcds - 1) / kXcds) * qchunks) : dim3(pblocks, qchunks);
+static inline dim3 tile_grid(int pblocks, int qsplit, int xcd_map) {
+  return xcd_map ? dim3(kXcds * ((pblocks + kXcds - 1) / kXcds) * qsplit) : dim3(pblocks, qsplit);
 }
 
-template <class Rec, int MODE, int T, int COMP>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(T == 1 && MODE != kModeHess ? 8 : 1, 8))) void k_pairs(
-    const Rec *__restrict__ P, int nP, const Rec *__restrict__ Q, int nQ,
-    int qchunk, int pblocks, int qchunks, int xcd_map, double *__restrict__ out, double t0, double t1,
-    double t2) {
+struct NearArg {
+  const int *ordP;    // stationary points' Hilbert order
+  const float *lamP;  // and their lam (times lam_scale: bound for the transformed ones)
+  float lam_scale;
+  const int *ordQ;    // streamed points' index
+  const QAux *auxQ;
+  const QBox *boxQ;
+  int nP, nQ, pblocks, qsplit, xcd_map;
+  int qchunk, gpc, ngroups;  // groups: gpc per chunk of qchunk streamed points
+  int win;                   // groups per window
+};
+
+// Lane k of the own row of 16, as an operand (k a constant).
+template <int K>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xF, 0xF, true));
+}
+template <int K>
+__device__ __forceinline__ void row_bcast(const Rec3F &q, Rec3F &r) {
+  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy); r.hz = row_bcast<K>(q.hz);
+  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly); r.lz = row_bcast<K>(q.lz);
+  r.s11 = row_bcast<K>(q.s11); r.s22 = row_bcast<K>(q.s22); r.s33 = row_bcast<K>(q.s33);
+  r.s12 = row_bcast<K>(q.s12); r.s13 = row_bcast<K>(q.s13); r.s23 = row_bcast<K>(q.s23);
+}
+template <int K>
+__device__ __forceinline__ void row_bcast(const Rec3I &q, Rec3I &r) {
+  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy); r.hz = row_bcast<K>(q.hz);
+  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly); r.lz = row_bcast<K>(q.lz);
+  r.s = row_bcast<K>(q.s);
+}
+template <int K>
+__device__ __forceinline__ void row_bcast(const Rec2F &q, Rec2F &r) {
+  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy);
+  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly);
+  r.s11 = row_bcast<K>(q.s11); r.s12 = row_bcast<K>(q.s12); r.s22 = row_bcast<K>(q.s22);
+}
+template <int K>
+__device__ __forceinline__ void row_bcast(const Rec2I &q, Rec2I &r) {
+  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy);
+  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly);
+  r.s = row_bcast<K>(q.s);
+}
+
+// The FP32 sums of a group go to the FP64 ones.
+template <int NA>
+__device__ __forceinline__ void flush_group(float *acc, double *dacc) {
+#pragma unroll
+  for (int a = 0; a < NA; ++a) {
+    dacc[a] += (double)acc[a];
+    acc[a] = 0.0f;
+  }
+}
+
+// Pairs of entries K..15 (below n) of the 16 records that each row holds;
+// bit k of first: entry k opens a group.
+template <class Rec, int MODE, int COMP, int NA, int K>
+__device__ __forceinline__ void eval_rows(const Rec &p, const Rec &q, unsigned first, int n, float *acc,
+                                          double *dacc) {
+  if constexpr (K < 16) {
+    if (K >= n) return;  // uniform
+    if ((first >> K) & 1u) flush_group<NA>(acc, dacc);
+    Rec r;
+    row_bcast<K>(q, r);
+    pair_eval<MODE, COMP>(p, r, acc);
+    eval_rows<Rec, MODE, COMP, NA, K + 1>(p, q, first, n, acc, dacc);
+  }
+}
+
+// Inclusive prefix sum over the 64 lanes.
+__device__ __forceinline__ int wave_scan(int v, int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(v, d, 64);
+    if (lane >= d) v += u;
+  }
+  return v;
+}
+
+// The pairs of the set bits of the lanes' groups (lane's group: 64 bits, first
+// streamed point js), group by group in lane order: listed in rounds of whole
+// groups, at most kCap entries (a group has at most 64).
+template <class Rec, int MODE, int COMP, int NA>
+__device__ __forceinline__ void walk_groups(const Rec &p, const Rec *__restrict__ Q, unsigned *list, int lane,
+                                            unsigned mlo, unsigned mhi, int js, double *dacc) {
+  const int cnt = __popc(mlo) + __popc(mhi);
+  const int incl = wave_scan(cnt, lane), excl = incl - cnt;
+  const int total = __builtin_amdgcn_readlane(incl, 63);
+  for (int done = 0; done < total;) {
+    const bool in = cnt > 0 && excl >= done && incl - done <= kCap;
+    if (in) {
+      unsigned *e = list + (excl - done);
+      unsigned flag = 1u << 31;  // opens a group
+      for (unsigned m = mlo; m; m &= m - 1) {
+        *e++ = (unsigned)(js + __builtin_ctz(m)) | flag;
+        flag = 0u;
+      }
+      for (unsigned m = mhi; m; m &= m - 1) {
+        *e++ = (unsigned)(js + 32 + __builtin_ctz(m)) | flag;
+        flag = 0u;
+      }
+    }
+    const int last = 63 - __builtin_clzll(__ballot(in));
+    const int n = __builtin_amdgcn_readlane(incl, last) - done;
+    done += n;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float acc[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
+    for (int e0 = 0; e0 < n; e0 += 16) {
+      const unsigned e = list[min(e0 + (lane & 15), n - 1)];
+      const Rec q = Q[e & 0x7fffffffu];
+      unsigned first = (unsigned)__ballot((int)e < 0) & 0xffffu;
+      if (e0 == 0) first &= ~1u;  // the sums are 0
+      eval_rows<Rec, MODE, COMP, NA, 0>(p, q, first, n - e0, acc, dacc);
+    }
+    flush_group<NA>(acc, dacc);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// One chunk of the Hessian pass is done: its energy and pose gradient go to r,
+// EW, B (FP32, as summed) and x' - t to the point's record of this chunk, and
+// the sums start again.  The transformed sources are stationary, so d = x' - y
+// flips the sign of EW and, for pose_contrib, of B (see the epilogue).
+constexpr int kHessRec = 12;
+template <class Rec, int NA>
+__device__ __forceinline__ void hess_chunk(const Rec &p, double *dacc, const double *t, double *r,
+                                           float *__restrict__ out, int pi) {
   using Tr = RecTraits<Rec>;
+  dacc[0] *= Tr::ESCALE;
+#pragma unroll
+  for (int a = 1; a < NA; ++a) dacc[a] *= -Tr::GSCALE;
+  if (pi >= 0) {
+    pose_contrib(p, dacc, t, r);
+    float v[kHessRec];
+#pragma unroll
+    for (int u = 1; u < 4; ++u) v[u - 1] = -(float)dacc[u];
+    // isotropic records: B = P - Q I
+    const float qd = Tr::FULL ? 0.0f : (float)dacc[NA - 1];
+#pragma unroll
+    for (int u = 4; u < 10; ++u)
+      v[u - 1] = Tr::FULL ? -(float)dacc[u] : -((float)dacc[u] - ((u == 4 || u == 7 || u == 9) ? qd : 0.0f));
+    v[9] = (float)((double)p.hx + (double)p.lx - t[0]);
+    v[10] = (float)((double)p.hy + (double)p.ly - t[1]);
+    v[11] = (float)((double)p.hz + (double)p.lz - t[2]);
+    float4 *o = reinterpret_cast<float4 *>(out + (size_t)pi * kHessRec);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) o[q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+  }
+#pragma unroll
+  for (int a = 0; a < NA; ++a) dacc[a] = 0.0;
+}
+
+// The Hessian entries of one tile -- 256 T stationary points, in kept order, of
+// one chunk -- summed as the point records say: FP32 over a wave's 64 T points,
+// then FP64.  Workgroup g takes tiles g, g + gridDim.x, ... and writes its 21
+// sums to out.
+__global__ __launch_bounds__(kBlock) void k_hess_tiles(const float *__restrict__ rec, int nP, int T, int tiles_p,
+                                                       int tiles, double *__restrict__ out) {
+  __shared__ float hred[kBlock / 64][21];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double sum = 0.0;
+  for (int tl = blockIdx.x; tl < tiles; tl += gridDim.x) {
+    const int c = tl / tiles_p, pb = tl - c * tiles_p;
+    const int base = pb * (kBlock * T) + wave * (64 * T) + lane;
+    float h[21];
+#pragma unroll
+    for (int q = 0; q < 21; ++q) h[q] = 0.0f;
+    for (int k = 0; k < T; ++k) {
+      const int pi = base + 64 * k;
+      if (pi >= nP) continue;
+      const float4 *v = reinterpret_cast<const float4 *>(rec + ((size_t)c * nP + pi) * kHessRec);
+      const float4 u0 = v[0], u1 = v[1], u2 = v[2];
+      const float a[10] = {0.0f, u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w, u2.x};
+      const float z[3] = {u2.y, u2.z, u2.w};
+      int q = 0;
+#pragma unroll
+      for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = i; j < 6; ++j) h[q++] += point_hessian_entry(i, j, z, a);
+    }
+    __syncthreads();  // the last tile's sums have been read
+#pragma unroll
+    for (int q = 0; q < 21; ++q) {
+      const float v = wave_sum_f(h[q]);
+      if (lane == 0) hred[wave][q] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 21) {
+#pragma unroll
+      for (int w = 0; w < kBlock / 64; ++w) sum += (double)hred[w][threadIdx.x];
+    }
+  }
+  if (threadIdx.x < 21) out[(size_t)blockIdx.x * kHessPart + threadIdx.x] = sum;
+}
+
+template <class Rec>
+__device__ __forceinline__ void stat_pos(const Rec &r, float *x) {
+  x[0] = r.hx;
+  x[1] = r.hy;
+  if constexpr (RecTraits<Rec>::D == 3)
+    x[2] = r.hz;
+  else
+    x[2] = 0.0f;
+}
+
+template <class Rec, int MODE, int COMP, bool XSRC>
+__global__ __launch_bounds__(kNearBlock) __attribute__((amdgpu_waves_per_eu(MODE == kModeHess || (MODE != kModeEnergy && RecTraits<Rec>::FULL) ? 6 : 8, 8))) void k_near(
+    const void *__restrict__ Pv, const Rec *__restrict__ Q, NearArg na, PoseArg ps, double *__restrict__ out,
+    float *__restrict__ hess) {
+  using Tr = RecTraits<Rec>;
+  constexpr int D = Tr::D;
   constexpr bool GRAD = MODE != kModeEnergy;
   // the Hessian pass needs B: isotropic records then hold it in two parts
-  constexpr int NA = MODE == kModeHess ? (Tr::FULL ? Tr::NACC : 11) : (GRAD ? Tr::NACC : 1);
-  constexpr int PART = MODE == kModeHess ? kHessPart : kPosePart;
+  // (the pose pass needs no G)
+  constexpr int NA = MODE == kModeHess                ? (Tr::FULL ? Tr::NACC : 11)
+                     : MODE == kModePose && !Tr::FULL ? 1 + D
+                     : GRAD                           ? Tr::NACC
+                                                      : 1;
+  // per wave kCap list entries, then the window's groups, 64 bits each; later
+  // the epilogue's staging
+  extern __shared__ unsigned s_dyn[];
+  unsigned *const s_bits = s_dyn + kNearWaves * kCap;
+  __shared__ Rec s_p[64];
+  __shared__ QBox s_row[kRows], s_quad[kQuads];
   int sb, qc;
-  if (!xcd_tile(pblocks, qchunks, xcd_map, &sb, &qc)) return;  // grid padding (whole workgroup)
+  if (!xcd_tile(na.pblocks, na.qsplit, na.xcd_map, &sb, &qc)) return;  // grid padding (whole workgroup)
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int pbase = sb * (kBlock * T) + wave * (64 * T) + lane;
-  const int q0 = qc * qchunk;
-  const int q1 = min(q0 + qchunk, nQ);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ppos = sb * 64 + lane;  // Hilbert position of the lane's point
+  const bool valid = ppos < na.nP;
 
-  Rec p[T];
+  if (wave == 0) {
+    const int pp = min(ppos, na.nP - 1);
+    const int pi = na.ordP[pp];
+    Rec r;
+    if constexpr (XSRC)
+      transform_rec(reinterpret_cast<const double *>(Pv) + (size_t)pi * (D + D * D), ps, r);
+    else
+      r = reinterpret_cast<const Rec *>(Pv)[pi];
+    s_p[lane] = r;
+    float x[3];
+    stat_pos(r, x);
+    QBox b, b4;
 #pragma unroll
-  for (int k = 0; k < T; ++k) p[k] = P[min(pbase + 64 * k, nP - 1)];
-
-  double dacc[T][NA];
-#pragma unroll
-  for (int k = 0; k < T; ++k)
-#pragma unroll
-    for (int a = 0; a < NA; ++a) dacc[k][a] = 0.0;
-
-  // the streamed records are software-pipelined two deep: record j + 2 is
-  // requested while record j is used (q0 < q1 for every workgroup; indices
-  // clamped to the chunk)
-  Rec qa = Q[q0], qb = Q[min(q0 + 1, q1 - 1)];
-  for (int j0 = q0; j0 < q1; j0 += kSub) {
-    float acc[T][NA];
-#pragma unroll
-    for (int k = 0; k < T; ++k)
-#pragma unroll
-      for (int a = 0; a < NA; ++a) acc[k][a] = 0.0f;
-    const int j1 = min(j0 + kSub, q1);
-#pragma unroll 2
-    for (int j = j0; j < j1; ++j) {
-      const Rec q = qa;
-      qa = qb;
-      qb = Q[min(j + 2, q1 - 1)];
-#pragma unroll
-      for (int k = 0; k < T; ++k) pair_eval<MODE, COMP>(p[k], q, acc[k]);
+    for (int a = 0; a < 3; ++a) {
+      const float lo4 = quad_min(x[a]), hi4 = quad_max(x[a]);
+      const float lo = row_min(x[a]), hi = row_max(x[a]);
+      const float slack = 2.4e-7f * fmaxf(fabsf(lo), fabsf(hi));  // the lo parts
+      b.lo[a] = lo - slack;
+      b.hi[a] = hi + slack;
+      b4.lo[a] = lo4 - slack;
+      b4.hi[a] = hi4 + slack;
     }
+    const float lam = na.lamP[pp] * na.lam_scale;
+    b.lam = row_max(lam);
+    b4.lam = quad_max(lam);
+    b.pad = b4.pad = 0.0f;
+    if ((lane & 3) == 0) s_quad[lane >> 2] = b4;
+    if ((lane & 15) == 0) s_row[lane >> 4] = b;
+  }
+
+  Rec p;
+  double dacc[NA];
 #pragma unroll
-    for (int k = 0; k < T; ++k)
+  for (int a = 0; a < NA; ++a) dacc[a] = 0.0;
+  double r[kPosePart];  // [E, rotation, translation]
 #pragma unroll
-      for (int a = 0; a < NA; ++a) dacc[k][a] += (double)acc[k][a];
+  for (int a = 0; a < kPosePart; ++a) r[a] = 0.0;
+
+  unsigned *const list = s_dyn + wave * kCap;
+  const int nbox = (na.nQ + 63) >> 6;
+  for (int w0 = 0; w0 < na.ngroups; w0 += na.win) {
+    const int wn = min(na.win, na.ngroups - w0);
+    if (w0 > 0) __syncthreads();  // the last window's bits have been read
+    for (int i = threadIdx.x; i < 2 * wn; i += kNearBlock) s_bits[i] = 0u;
+    __syncthreads();
+    if (w0 == 0) p = s_p[lane];
+    // boxes are dealt to the waves one by one: near ones follow each other
+    for (int b0 = wave; b0 < nbox; b0 += kNearBlock) {
+      const int bl = b0 + lane * kNearWaves;
+      bool hit = false;
+      if (bl < nbox) {
+        const QBox q = na.boxQ[bl];
+#pragma unroll
+        for (int k = 0; k < kRows; ++k)
+          hit = hit || box_near(s_row[k], q.lo[0], q.lo[1], q.lo[2], q.hi[0], q.hi[1], q.hi[2], q.lam);
+      }
+      for (unsigned long long m = __ballot(hit); m; m &= m - 1) {
+        asm volatile("" ::: "memory");
+        const int i = (b0 + __builtin_ctzll(m) * kNearWaves) * 64 + lane;
+        if (i >= na.nQ) continue;
+        const QAux q = na.auxQ[i];
+        const int j = na.ordQ[i];
+        unsigned rows = 0;
+#pragma unroll
+        for (int k = 0; k < kRows; ++k)
+          rows |= box_near(s_row[k], q.x, q.y, q.z, q.x, q.y, q.z, q.lam) ? 1u << k : 0u;
+        bool near = false;
+        asm volatile("" ::: "memory");  // the boxes stay in LDS (hoisted, their 160 words would spill)
+        if (rows)
+#pragma unroll
+          for (int k = 0; k < kQuads; ++k) near = near || box_near(s_quad[k], q.x, q.y, q.z, q.x, q.y, q.z, q.lam);
+        if (!near) continue;
+        const int c = j / na.qchunk, r = j - c * na.qchunk;
+        const int g = c * na.gpc + (r >> 6) - w0;
+        if (g >= 0 && g < wn) atomicOr(&s_bits[2 * g + ((r >> 5) & 1)], 1u << (r & 31));
+      }
+    }
+    __syncthreads();
+    if constexpr (MODE == kModeHess) {
+      // chunk c goes whole to part c % qsplit, wave (c / qsplit) % 8; its
+      // sums leave for k_hess_tiles when its last group is done
+      const int gend = w0 + wn;
+      for (int c = na.qsplit * wave + qc; c * na.gpc < gend; c += na.qsplit * kNearWaves) {
+        if ((c + 1) * na.gpc <= w0) continue;
+        const int c1 = min((c + 1) * na.gpc, gend);
+        for (int gb = max(c * na.gpc, w0); gb < c1; gb += 64) {
+          const int g = gb + lane;
+          const bool own = g < c1;
+          walk_groups<Rec, MODE, COMP, NA>(p, Q, list, lane, own ? s_bits[2 * (g - w0)] : 0u,
+                                           own ? s_bits[2 * (g - w0) + 1] : 0u,
+                                           c * na.qchunk + (g - c * na.gpc) * 64, dacc);
+        }
+        if ((c + 1) * na.gpc > gend) break;  // goes on in the next window
+        hess_chunk<Rec, NA>(p, dacc, ps.t, r, hess + (size_t)c * na.nP * kHessRec, valid ? na.ordP[ppos] : -1);
+      }
+    } else {
+      // group g goes to part g % qsplit, wave (g / qsplit) % 8
+      for (int g0 = 0; g0 < wn; g0 += kNearBlock * na.qsplit) {
+        const int g = g0 + (lane * kNearWaves + wave) * na.qsplit + qc;
+        const bool own = g < wn;
+        const int c = (w0 + g) / na.gpc;
+        walk_groups<Rec, MODE, COMP, NA>(p, Q, list, lane, own ? s_bits[2 * g] : 0u, own ? s_bits[2 * g + 1] : 0u,
+                                         c * na.qchunk + (w0 + g - c * na.gpc) * 64, dacc);
+      }
+    }
   }
 
   // Isotropic records: variances were times ln 4 (ESCALE, GSCALE).  A pose
@@ -170,122 +574,70 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(T == 1 &
   // gradient is then taken about the sources, whose rotation also turns
   // their covariances.  With EW and B both negated, pose_contrib's
   // (p - t) x EW + vee(S_p B - B S_p) is exactly that gradient.
-  constexpr bool kSwapped = (MODE == kModePose || MODE == kModeHess) && COMP == 2;
-  if (!RecTraits<Rec>::FULL || kSwapped) {
+  constexpr bool kSwapped = MODE == kModePose && COMP == 2;
+  if (MODE != kModeHess && (!RecTraits<Rec>::FULL || kSwapped)) {
     constexpr double gs = kSwapped ? -RecTraits<Rec>::GSCALE : RecTraits<Rec>::GSCALE;
+    dacc[0] *= RecTraits<Rec>::ESCALE;
 #pragma unroll
-    for (int k = 0; k < T; ++k) {
-      dacc[k][0] *= RecTraits<Rec>::ESCALE;
-#pragma unroll
-      for (int a = 1; a < NA; ++a) dacc[k][a] *= gs;
-    }
+    for (int a = 1; a < NA; ++a) dacc[a] *= gs;
   }
 
-  if (MODE == kModePoint) {
+  double *stage = reinterpret_cast<double *>(s_dyn);
+  if constexpr (MODE == kModePoint) {
+    // the 8 waves' sums of each point, in wave order, kHalf values at a time
+    constexpr int kHalf = (NA + 1) / 2;
 #pragma unroll
-    for (int k = 0; k < T; ++k) {
-      const int pi = pbase + 64 * k;
-      if (pi < nP) {
-        double *o = out + ((size_t)qc * nP + pi) * NA;
+    for (int h = 0; h < 2; ++h) {
+      const int nv = h == 0 ? kHalf : NA - kHalf;
+      __syncthreads();
 #pragma unroll
-        for (int a = 0; a < NA; ++a) o[a] = dacc[k][a];
+      for (int a = 0; a < nv; ++a) stage[(wave * kHalf + a) * 64 + lane] = dacc[h * kHalf + a];
+      __syncthreads();
+      for (int e = threadIdx.x; e < 64 * nv; e += kNearBlock) {
+        const int k = e / nv, a = e - k * nv;
+        if (sb * 64 + k < na.nP) {
+          double s = stage[a * 64 + k];
+#pragma unroll
+          for (int w = 1; w < kNearWaves; ++w) s += stage[(w * kHalf + a) * 64 + k];
+          out[((size_t)qc * na.nP + na.ordP[sb * 64 + k]) * NA + h * kHalf + a] = s;
+        }
       }
     }
     return;
   }
 
-  double r[kPosePart];
-#pragma unroll
-  for (int a = 0; a < kPosePart; ++a) r[a] = 0.0;
-  const double tt[3] = {t0, t1, t2};
-#pragma unroll
-  for (int k = 0; k < T; ++k) {
-    if (pbase + 64 * k < nP) {
-      if (GRAD)
-        pose_contrib(p[k], dacc[k], tt, r);
-      else
-        r[0] += dacc[k][0];
-    }
+  if (MODE != kModeHess && valid) {
+    if constexpr (GRAD)
+      pose_contrib(p, dacc, ps.t, r);
+    else
+      r[0] += dacc[0];
   }
-  double *o = out + ((size_t)qc * pblocks + sb) * PART;
+  double *o = out + ((size_t)qc * na.pblocks + sb) * kPosePart;
+  __syncthreads();  // the bits have been read
   if (GRAD) {
     // Workgroup sums of the kPosePart values in a fixed order: every lane's
-    // values go to LDS; thread (a, k) = (tid / 32, tid % 32) adds entries
-    // k, k + 32, ..., k + 224 of value a (consecutive lanes read consecutive
-    // doubles: no bank conflict); each half wave then sums its 32 partials
-    // (DPP row rotations, then the two row sums), value 2 * wave in the low
-    // half and 2 * wave + 1 in the high half.
-    static_assert(kPosePart * 32 == kBlock, "one half wave per pose value");
-    __shared__ double stage[kPosePart][kBlock];
+    // values go to LDS; wave a adds entries lane, lane + 64, ... of value a
+    // (consecutive lanes read consecutive doubles: no bank conflict), then
+    // sums over its lanes by DPP.
+    static_assert(kPosePart == kNearWaves, "one wave per pose value");
 #pragma unroll
-    for (int a = 0; a < kPosePart; ++a) stage[a][threadIdx.x] = r[a];
+    for (int a = 0; a < kPosePart; ++a) stage[a * kNearBlock + threadIdx.x] = r[a];
     __syncthreads();
-    const int a = threadIdx.x >> 5, k = threadIdx.x & 31;
     double s = 0.0;
 #pragma unroll
-    for (int i = 0; i < kBlock / 32; ++i) s += stage[a][k + 32 * i];
-    double lo, hi;
-    half_wave_sums(s, lo, hi);
-    if (lane == 0) {
-      o[2 * wave] = lo;
-      o[2 * wave + 1] = hi;
-    }
-    if constexpr (MODE == kModeHess && Tr::D == 3) {
-      // the Hessian entries, one at a time: lane sums over its T points, a
-      // wave sum, then the waves' sums in order.  The block above negated
-      // EW and B (sources stationary); the entries need them as summed.
-      constexpr float sg = kSwapped ? -1.0f : 1.0f;
-      __shared__ float hred[kBlock / 64][21];
-      int q = 0;
-#pragma unroll
-      for (int i = 0; i < 6; ++i)
-#pragma unroll
-        for (int j = i; j < 6; ++j) {
-          float v = 0.0f;
-#pragma unroll
-          for (int kk = 0; kk < T; ++kk) {
-            if (pbase + 64 * kk >= nP) continue;
-            float av[10];
-            av[0] = 0.0f;
-#pragma unroll
-            for (int u = 1; u < 4; ++u) av[u] = sg * (float)dacc[kk][u];
-            if (Tr::FULL) {
-#pragma unroll
-              for (int u = 4; u < 10; ++u) av[u] = sg * (float)dacc[kk][u];
-            } else {  // B = P - Q I
-              const float qd = (float)dacc[kk][NA - 1];
-#pragma unroll
-              for (int u = 4; u < 10; ++u)
-                av[u] = sg * ((float)dacc[kk][u] - ((u == 4 || u == 7 || u == 9) ? qd : 0.0f));
-            }
-            const float z[3] = {(float)((double)p[kk].hx + (double)p[kk].lx - t0),
-                                (float)((double)p[kk].hy + (double)p[kk].ly - t1),
-                                (float)((double)p[kk].hz + (double)p[kk].lz - t2)};
-            v += point_hessian_entry(i, j, z, av);
-          }
-          v = wave_sum_f(v);
-          if (lane == 0) hred[wave][q] = v;
-          ++q;
-        }
-      __syncthreads();
-      if (threadIdx.x < 21) {
-        double s2 = 0.0;
-#pragma unroll
-        for (int w = 0; w < kBlock / 64; ++w) s2 += (double)hred[w][threadIdx.x];
-        o[kPosePart + threadIdx.x] = s2;
-      }
-    }
+    for (int i = 0; i < kNearWaves; ++i) s += stage[wave * kNearBlock + lane + 64 * i];
+    s = wave_sum(s);
+    if (lane == 0) o[wave] = s;
   } else {
-    r[0] = wave_sum(r[0]);
-    __shared__ double red[kBlock / 64];
-    if (lane == 0) red[wave] = r[0];
+    const double v = wave_sum(r[0]);
+    if (lane == 0) stage[wave] = v;
     __syncthreads();
     if (threadIdx.x < kPosePart) {
       double s = 0.0;
       if (threadIdx.x == 0) {
-        s = red[0];
+        s = stage[0];
 #pragma unroll
-        for (int w = 1; w < kBlock / 64; ++w) s += red[w];
+        for (int w = 1; w < kNearWaves; ++w) s += stage[w];
       }
       o[threadIdx.x] = s;
     }
@@ -329,36 +681,24 @@ __global__ __launch_bounds__(kBlock) void k_reduce_parts(
   }
 }
 
-// The Hessian pass's partials (kHessPart doubles per workgroup of the pair
-// kernel, 29 used): workgroup g sums its contiguous range, each thread over
-// whole records, then the 256 threads' values value by value through LDS in
-// a fixed tree order; the host adds the workgroups' sums in order.
-constexpr int kHessGroups = 64;
-constexpr int kHessUsed = kPosePart + 21;
-__global__ __launch_bounds__(kBlock) void k_reduce_hess(const double *__restrict__ parts, int nparts,
-                                                        double *__restrict__ res) {
-  const int len = (nparts + (int)gridDim.x - 1) / (int)gridDim.x;
-  const int q0 = blockIdx.x * len, q1 = min(q0 + len, nparts);
-  double s[kHessUsed];
-#pragma unroll
-  for (int a = 0; a < kHessUsed; ++a) s[a] = 0.0;
-  for (int q = q0 + (int)threadIdx.x; q < q1; q += kBlock) {
-    const double *row = parts + (size_t)q * kHessPart;
-#pragma unroll
-    for (int a = 0; a < kHessUsed; ++a) s[a] += row[a];
-  }
-  __shared__ double stage[kBlock];
-#pragma unroll 1
-  for (int a = 0; a < kHessUsed; ++a) {
-    stage[threadIdx.x] = s[a];
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) stage[threadIdx.x] += stage[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) res[kHessPart * blockIdx.x + a] = stage[0];
-    __syncthreads();
-  }
+// The 21 Hessian sums of k_hess_tiles' workgroups (kHessPart doubles each), in a
+// fixed order: thread (a, k) adds records k, k + 32, ... of entry a, then each
+// half wave sums its 32.
+constexpr int kHessGroups = 512;
+__global__ __launch_bounds__(1024) void k_reduce_hess(const double *__restrict__ parts, int nparts,
+                                                      double *__restrict__ res) {
+  const int a = threadIdx.x & 31, k = threadIdx.x >> 5;
+  __shared__ double stage[32][33];
+  double s = 0.0;
+  if (a < 21)
+    for (int q = k; q < nparts; q += 32) s += parts[(size_t)q * kHessPart + a];
+  stage[a][k] = s;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double lo, hi;
+  half_wave_sums(stage[2 * wave + (lane >> 5)][lane & 31], lo, hi);
+  if (lane == 0 && 2 * wave < 21) res[2 * wave] = lo;
+  if (lane == 0 && 2 * wave + 1 < 21) res[2 * wave + 1] = hi;
 }
 
 // Per-point sums over streamed chunks, in chunk order.
@@ -374,96 +714,16 @@ __global__ __launch_bounds__(kBlock) void k_reduce_points(
 }
 
 // ---------------------------------------------------------------------------
-// Per-call source records: x' = R x + t and S' = R S R^T in FP64, then
-// split to FP32 hi/lo (positions) and rounded (covariance).
-// ---------------------------------------------------------------------------
-template <int D, bool ISO>
-__global__ __launch_bounds__(kBlock) void k_transform_src(
-    const double *__restrict__ src, int n, PoseArg ps, void *__restrict__ outv) {
-  const int k = blockIdx.x * kBlock + threadIdx.x;
-  if (k >= n) return;
-  const double *s = src + (size_t)k * (D + D * D);
-  double xp[3];
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    double v = ps.t[a];
-#pragma unroll
-    for (int b = 0; b < D; ++b) v = fma(ps.R[a + D * b], s[b], v);
-    xp[a] = v;
-  }
-  float hi[3], lo[3];
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    hi[a] = (float)xp[a];
-    lo[a] = (float)(xp[a] - (double)hi[a]);
-  }
-  const double *S = s + D;
-  if (ISO) {
-    if (D == 3) {
-      Rec3I r;
-      r.hx = hi[0]; r.hy = hi[1]; r.hz = hi[2];
-      r.lx = lo[0]; r.ly = lo[1]; r.lz = lo[2];
-      r.s = (float)(S[0] * kLn4);
-      r.pad0 = 0.0f;
-      reinterpret_cast<Rec3I *>(outv)[k] = r;
-    } else {
-      Rec2I r;
-      r.hx = hi[0]; r.hy = hi[1]; r.lx = lo[0]; r.ly = lo[1];
-      r.s = (float)(S[0] * kLn4);
-      r.pad0 = r.pad1 = r.pad2 = 0.0f;
-      reinterpret_cast<Rec2I *>(outv)[k] = r;
-    }
-    return;
-  }
-  // S' = R S R^T
-  double RS[9], Sp[9];
-#pragma unroll
-  for (int a = 0; a < D; ++a)
-#pragma unroll
-    for (int c = 0; c < D; ++c) {
-      double v = 0.0;
-#pragma unroll
-      for (int b = 0; b < D; ++b) v = fma(ps.R[a + D * b], S[b + D * c], v);
-      RS[a + D * c] = v;
-    }
-#pragma unroll
-  for (int a = 0; a < D; ++a)
-#pragma unroll
-    for (int c = 0; c < D; ++c) {
-      double v = 0.0;
-#pragma unroll
-      for (int b = 0; b < D; ++b) v = fma(RS[a + D * b], ps.R[c + D * b], v);
-      Sp[a + D * c] = v;
-    }
-  if (D == 3) {
-    Rec3F r;
-    r.hx = hi[0]; r.hy = hi[1]; r.hz = hi[2];
-    r.lx = lo[0]; r.ly = lo[1]; r.lz = lo[2];
-    r.s11 = (float)Sp[0];
-    r.s22 = (float)Sp[4];
-    r.s33 = (float)Sp[8];
-    r.s12 = (float)(0.5 * (Sp[3] + Sp[1]));
-    r.s13 = (float)(0.5 * (Sp[6] + Sp[2]));
-    r.s23 = (float)(0.5 * (Sp[7] + Sp[5]));
-    r.pad0 = r.pad1 = r.pad2 = r.pad3 = 0.0f;
-    reinterpret_cast<Rec3F *>(outv)[k] = r;
-  } else {
-    Rec2F r;
-    r.hx = hi[0]; r.hy = hi[1]; r.lx = lo[0]; r.ly = lo[1];
-    r.s11 = (float)Sp[0];
-    r.s22 = (float)Sp[3];
-    r.s12 = (float)(0.5 * (Sp[2] + Sp[1]));
-    r.pad0 = 0.0f;
-    reinterpret_cast<Rec2F *>(outv)[k] = r;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Launch planning
 // ---------------------------------------------------------------------------
 struct Plan {
-  int T = 1;
-  int pblocks = 1, qchunks = 1, qchunk = 1;
+  // Sub-tiles: chunks of qchunk streamed points, each cut into groups of kSub
+  // from its start.  They fix how the FP32 sums are grouped.
+  int qchunk = 1, gpc = 1, ngroups = 1;
+  int T = 1, tiles_p = 1, qchunks = 1;  // chunk tiles: tiles_p times 256 T stationary points, qchunks chunks
+  // Launch: pblocks workgroups of 64 stationary points times qsplit parts of
+  // the groups.
+  int pblocks = 1, qsplit = 1;
 };
 
 static int env_int(const char *name, int dflt) {
@@ -471,74 +731,100 @@ static int env_int(const char *name, int dflt) {
   return (v && *v) ? atoi(v) : dflt;
 }
 
-// Launch shape: T stationary points per lane and a target number of waves
-// (streamed chunks are sized to reach it).  A context may carry tuned values
-// (dugma_autotune); otherwise: T = 2 and 4096 waves, 16384 for very large
-// problems, so the grid covers the 256 CUs several times.
-static Plan make_plan(int nP, int nQ, int mode, int T, int target_waves, int max_chunks = 64) {
+// Waves a launch aims at when the stationary points alone give fewer: 4 per
+// SIMD of the 256 CUs.
+constexpr int kLaunchWaves = 4096;
+
+// Chunks so that tiles of 256 T stationary points x one chunk make about
+// target_waves waves, each chunk at least kMinChunk points.
+static Plan make_plan(int nP, int nQ, int mode, int T, int target_waves, int launch_waves, int max_chunks = 64) {
   Plan pl;
-  pl.T = T;
-  pl.pblocks = (nP + kBlock * T - 1) / (kBlock * T);
-  const int waves_p = pl.pblocks * (kBlock / 64);
+  const int tiles_p = (nP + kBlock * T - 1) / (kBlock * T);
+  const int waves_p = tiles_p * (kBlock / 64);
   int qc = (target_waves + waves_p - 1) / waves_p;
   int maxc = (nQ + kMinChunk - 1) / kMinChunk;
   if (mode == kModePoint) maxc = std::min(maxc, max_chunks);
-  // grid limits: 65,535 chunks on the 2-D grid, 2^31 - 1 threads on the
-  // padded 1-D (XCD-mapped) one
-  maxc = std::min({maxc, 65535, (int)(INT32_MAX / kBlock / (pl.pblocks + kXcds))});
+  maxc = std::min({maxc, 65535, (int)(INT32_MAX / kBlock / (tiles_p + kXcds))});
   qc = std::max(1, std::min(qc, maxc));
   pl.qchunk = (nQ + qc - 1) / qc;
+  pl.T = T;
+  pl.tiles_p = tiles_p;
   pl.qchunks = (nQ + pl.qchunk - 1) / pl.qchunk;
+  pl.gpc = (pl.qchunk + kSub - 1) / kSub;
+  pl.ngroups = pl.qchunks * pl.gpc;
+  pl.pblocks = (nP + 63) / 64;
+  const int waves = pl.pblocks * kNearWaves;
+  pl.qsplit = std::max(1, std::min((launch_waves + waves - 1) / waves, (pl.ngroups + kNearWaves - 1) / kNearWaves));
   return pl;
 }
 
+// Sub-tiles: T = 2 and 4096 waves, 16384 for very large problems (environment
+// overrides).  Launch: kLaunchWaves, or what dugma_autotune chose.
 static Plan ctx_plan(const dugma_ctx *c, int nP, int nQ, int mode, bool iso) {
   int T = 2, tw = ((double)nP * nQ >= 1e9) ? 16384 : 4096;
-  const dugma_ctx::Tuned &tu = c->tuned[mode == kModeEnergy ? 0 : 1][iso ? 1 : 0];
-  if (tu.target_waves > 0) {
-    T = tu.T;
-    tw = tu.target_waves;
-  }
   T = env_int("DUGMA_LANE_POINTS", T) == 1 ? 1 : 2;
   tw = env_int("DUGMA_TARGET_WAVES", tw);
-  return make_plan(nP, nQ, mode, T, tw);
+  const dugma_ctx::Tuned &tu = c->tuned[mode == kModeEnergy ? 0 : 1][iso ? 1 : 0];
+  return make_plan(nP, nQ, mode, T, tw, tu.target_waves > 0 ? tu.target_waves : kLaunchWaves);
 }
 
-template <class Rec, int MODE, int COMP>
-static void launch_pairs_c(const Plan &pl, const Rec *P, int nP, const Rec *Q, int nQ,
-                           double *out, const double *t, hipStream_t s) {
-  // the XCD tile order for clouds beyond one L2, except in the per-point
-  // passes (measured 2% slower with it there); DUGMA_XCD_ORDER=0 in the
+// A pass's two point sets: the stationary cloud is 0 (targets) or 1
+// (sources), the other one is streamed.
+struct Sets {
+  int stat;        // stationary cloud
+  const void *P;   // its records in kept order (null: transformed from the source data in the kernel)
+  const void *Q;   // streamed records in kept order
+  float lam_scale;
+};
+
+template <class Rec, int MODE, int COMP, bool XSRC>
+static void launch_near_x(dugma_ctx *c, const Plan &pl, const Sets &st, const PoseArg &ps, double *out,
+                          float *hess = nullptr) {
+  NearArg na;
+  const int nP = st.stat == 0 ? c->nT : c->nS, nQ = st.stat == 0 ? c->nS : c->nT;
+  const NearCloud &cp = c->near[st.stat], &cq = c->near[1 - st.stat];
+  na.ordP = cp.ord;
+  na.lamP = cp.lam;
+  na.lam_scale = st.stat == 0 ? 1.0f : st.lam_scale;
+  na.ordQ = cq.ord;
+  na.auxQ = cq.aux;
+  na.boxQ = cq.box;
+  na.nP = nP;
+  na.nQ = nQ;
+  na.pblocks = pl.pblocks;
+  na.qsplit = pl.qsplit;
+  // the XCD tile order for clouds beyond one L2; DUGMA_XCD_ORDER=0 in the
   // environment keeps the 2-D order (the sums are the same, bit for bit)
-  const int xcd_map = MODE != kModePoint && (size_t)(nP + nQ) * sizeof(Rec) > kXcdMapBytes &&
-                              env_int("DUGMA_XCD_ORDER", 1) != 0
-                          ? 1
-                          : 0;
-  const dim3 grid = tile_grid(pl.pblocks, pl.qchunks, xcd_map), block(kBlock);
-  const double t0 = t[0], t1 = t[1], t2 = (RecTraits<Rec>::D == 3) ? t[2] : 0.0;
-  if (pl.T == 2)
-    hipLaunchKernelGGL((k_pairs<Rec, MODE, 2, COMP>), grid, block, 0, s, P, nP, Q, nQ, pl.qchunk,
-                       pl.pblocks, pl.qchunks, xcd_map, out, t0, t1, t2);
-  else
-    hipLaunchKernelGGL((k_pairs<Rec, MODE, 1, COMP>), grid, block, 0, s, P, nP, Q, nQ, pl.qchunk,
-                       pl.pblocks, pl.qchunks, xcd_map, out, t0, t1, t2);
+  na.xcd_map = (size_t)(nP + nQ) * sizeof(Rec) > kXcdMapBytes && env_int("DUGMA_XCD_ORDER", 1) != 0 ? 1 : 0;
+  na.qchunk = pl.qchunk;
+  na.gpc = pl.gpc;
+  na.ngroups = pl.ngroups;
+  // windows of whole chunks for the Hessian pass (or parts of one chunk)
+  na.win = MODE == kModeHess && pl.gpc <= kWinGroups ? kWinGroups / pl.gpc * pl.gpc : kWinGroups;
+  constexpr size_t kStage = MODE == kModeEnergy ? sizeof(double) * kNearWaves
+                            : MODE == kModePoint ? sizeof(double) * kNearBlock * ((RecTraits<Rec>::NACC + 1) / 2)
+                                                 : sizeof(double) * kNearBlock * kPosePart;
+  const size_t lds =
+      std::max(kStage, sizeof(unsigned) * kNearWaves * kCap + (size_t)8 * std::min(pl.ngroups, kWinGroups));
+  const void *P = XSRC ? (const void *)c->dSsrc : st.P;
+  hipLaunchKernelGGL((k_near<Rec, MODE, COMP, XSRC>), tile_grid(pl.pblocks, pl.qsplit, na.xcd_map),
+                     dim3(kNearBlock), lds, c->stream, P, (const Rec *)st.Q, na, ps, out, hess);
 }
 
 // comp: 0 none, 1 streamed side carries the lo part, 2 stationary side does.
 template <class Rec>
-static void launch_pairs(int mode, int comp, const Plan &pl, const Rec *P,
-                         int nP, const Rec *Q, int nQ, double *out,
-                         const double *t, hipStream_t s) {
-#define DUGMA_L(M, C) launch_pairs_c<Rec, M, C>(pl, P, nP, Q, nQ, out, t, s)
+static void launch_near(dugma_ctx *c, int mode, int comp, const Plan &pl, const Sets &st, const PoseArg &ps,
+                        double *out) {
+#define DUGMA_L(M, C, X) launch_near_x<Rec, M, C, X>(c, pl, st, ps, out)
   if (mode == kModeEnergy) {
     // comp 2 in these passes: the transformed sources are stationary (see pose_pass)
-    if (comp == 2) DUGMA_L(kModeEnergy, 2); else if (comp == 1) DUGMA_L(kModeEnergy, 1); else DUGMA_L(kModeEnergy, 0);
+    if (comp == 2) DUGMA_L(kModeEnergy, 2, true); else if (comp == 1) DUGMA_L(kModeEnergy, 1, false); else DUGMA_L(kModeEnergy, 0, false);
   } else if (mode == kModePose) {
-    if (comp == 2) DUGMA_L(kModePose, 2); else if (comp == 1) DUGMA_L(kModePose, 1); else DUGMA_L(kModePose, 0);
+    if (comp == 2) DUGMA_L(kModePose, 2, true); else if (comp == 1) DUGMA_L(kModePose, 1, false); else DUGMA_L(kModePose, 0, false);
   } else {
-    if (comp == 1) DUGMA_L(kModePoint, 1);
-    else if (comp == 2) DUGMA_L(kModePoint, 2);
-    else DUGMA_L(kModePoint, 0);
+    if (comp == 1) DUGMA_L(kModePoint, 1, false);
+    else if (comp == 2) DUGMA_L(kModePoint, 2, false);
+    else DUGMA_L(kModePoint, 0, false);
   }
 #undef DUGMA_L
 }
@@ -553,23 +839,37 @@ static PoseArg make_pose(const dugma_ctx *c, const double *R, const double *t) {
   return ps;
 }
 
-static int transform_sources(dugma_ctx *c, const PoseArg &ps, bool iso) {
+// The transformed sources' records in kept order, with their index: for the
+// passes that stream them.
+static int transform_sources(dugma_ctx *c, const PoseArg &ps, bool iso, float lam_scale) {
   if (c->nS == 0) return DUGMA_OK;
   dim3 grid((c->nS + kBlock - 1) / kBlock), block(kBlock);
   void *out = iso ? c->dSrecI : c->dSrecF;
+#define DUGMA_T(R) hipLaunchKernelGGL(k_transform_src<R>, grid, block, 0, c->stream, c->dSsrc, c->nS, ps, (R *)out)
   if (c->D == 3) {
-    if (iso)
-      hipLaunchKernelGGL((k_transform_src<3, true>), grid, block, 0, c->stream, c->dSsrc, c->nS, ps, out);
-    else
-      hipLaunchKernelGGL((k_transform_src<3, false>), grid, block, 0, c->stream, c->dSsrc, c->nS, ps, out);
+    if (iso) DUGMA_T(Rec3I); else DUGMA_T(Rec3F);
   } else {
-    if (iso)
-      hipLaunchKernelGGL((k_transform_src<2, true>), grid, block, 0, c->stream, c->dSsrc, c->nS, ps, out);
-    else
-      hipLaunchKernelGGL((k_transform_src<2, false>), grid, block, 0, c->stream, c->dSsrc, c->nS, ps, out);
+    if (iso) DUGMA_T(Rec2I); else DUGMA_T(Rec2F);
   }
+#undef DUGMA_T
   DUGMA_HIP(hipGetLastError());
-  return DUGMA_OK;
+  return near_index_sources(c, iso, out, lam_scale);
+}
+
+// Bound of R's largest singular value squared (1 for a rotation): what R can
+// do to a covariance's largest eigenvalue.
+static float pose_lam_scale(int D, const double *R) {
+  double big = 0.0;
+  for (int a = 0; a < D; ++a) {
+    double row = 0.0;
+    for (int b = 0; b < D; ++b) {
+      double v = 0.0;
+      for (int k = 0; k < D; ++k) v += R[k + D * a] * R[k + D * b];
+      row += std::fabs(v);
+    }
+    big = std::max(big, row);
+  }
+  return (float)(big * 1.000001);
 }
 
 static int resolve_iso(dugma_ctx *c, int cov_mode, bool *iso) {
@@ -605,28 +905,28 @@ static int pose_pass(dugma_ctx *c, const double *R, const double *t, bool iso,
   const int width = mode == kModeEnergy ? 1 : (D == 3 ? 7 : 4);
   for (int a = 0; a < width; ++a) res[a] = 0.0;
   if (c->nT == 0 || c->nS == 0) return DUGMA_OK;
-  // everything the launches need is settled first, so that the three
-  // launches leave the host back to back (the transform takes ~3 us)
+  // everything the launches need is settled first, so that they leave the
+  // host back to back
   PoseArg ps = make_pose(c, R, t);
   // The passes keep the transformed sources (FP32 hi + lo) stationary and
   // stream the targets (exact in FP32): the lo correction is then an
   // operation on VGPRs only (COMP 2) instead of a second one on the streamed
-  // SGPRs (COMP 1).  E is symmetric in the two roles; the gradient sums
-  // change sign (kernel epilogue).  Without compensation the targets stay
-  // stationary (COMP 0).
+  // SGPRs (COMP 1), and the kernel transforms its own 64 sources.  E is
+  // symmetric in the two roles; the gradient sums change sign (kernel
+  // epilogue).  Without compensation the targets stay stationary (COMP 0).
   const bool swap = sources_stationary();
   const int comp = swap ? 2 : (comp_enabled() ? 1 : 0);
   Plan pl = swap ? ctx_plan(c, c->nS, c->nT, mode, iso) : ctx_plan(c, c->nT, c->nS, mode, iso);
-  const size_t nparts = (size_t)pl.pblocks * pl.qchunks;
+  const size_t nparts = (size_t)pl.pblocks * pl.qsplit;
   // few partials: the pair kernel writes them to pinned host memory and the
-  // host sums them after the sync; many: a device reduction launch
+  // host sums them as they arrive; many: a device reduction launch
   const bool host_sum = nparts <= (size_t)dugma_ctx::kHostParts;
   double *parts = c->dparts;
   int rc;
+  if (fixed_parts && std::max((size_t)pl.tiles_p * pl.qchunks, nparts) > fixed_records)
+    return fail(DUGMA_ERR_SIZE, "dugma_energy_grad_noalloc: the launch needs more partial records than the "
+                                "scratch array holds (lower DUGMA_TARGET_WAVES or the autotuned wave count)");
   if (!host_sum && fixed_parts) {
-    if (nparts > fixed_records)
-      return fail(DUGMA_ERR_SIZE, "dugma_energy_grad_noalloc: the launch needs more partial records than the "
-                                  "scratch array holds (lower DUGMA_TARGET_WAVES or the autotuned wave count)");
     parts = fixed_parts;
   } else if (!host_sum) {
     rc = c->part.ensure(nparts * kPosePart * sizeof(double));
@@ -634,23 +934,28 @@ static int pose_pass(dugma_ctx *c, const double *R, const double *t, bool iso,
     parts = (double *)c->part.ptr;
   }
   const int groups = (int)std::min<size_t>(kRedGroups, (nparts + kBlock - 1) / kBlock);
-  if (!host_sum) preset_slots(c->hres, kPosePart * groups);
-  rc = transform_sources(c, ps, iso);
-  if (rc) return rc;
+  const float lam_scale = pose_lam_scale(D, R);
+  if (host_sum)
+    preset_slots(c->hparts, (int)(kPosePart * nparts));
+  else
+    preset_slots(c->hres, kPosePart * groups);
+  if (!swap) {
+    rc = transform_sources(c, ps, iso, lam_scale);
+    if (rc) return rc;
+  }
   PairTimer timer(c);
   const void *tgt = iso ? c->dTrecI : c->dTrecF, *src = iso ? c->dSrecI : c->dSrecF;
-  const void *P = swap ? src : tgt, *Q = swap ? tgt : src;
-  const int nP = swap ? c->nS : c->nT, nQ = swap ? c->nT : c->nS;
+  const Sets st = {swap ? 1 : 0, swap ? nullptr : tgt, swap ? tgt : src, lam_scale};
   if (D == 3) {
     if (iso)
-      launch_pairs<Rec3I>(mode, comp, pl, (const Rec3I *)P, nP, (const Rec3I *)Q, nQ, parts, ps.t, c->stream);
+      launch_near<Rec3I>(c, mode, comp, pl, st, ps, parts);
     else
-      launch_pairs<Rec3F>(mode, comp, pl, (const Rec3F *)P, nP, (const Rec3F *)Q, nQ, parts, ps.t, c->stream);
+      launch_near<Rec3F>(c, mode, comp, pl, st, ps, parts);
   } else {
     if (iso)
-      launch_pairs<Rec2I>(mode, comp, pl, (const Rec2I *)P, nP, (const Rec2I *)Q, nQ, parts, ps.t, c->stream);
+      launch_near<Rec2I>(c, mode, comp, pl, st, ps, parts);
     else
-      launch_pairs<Rec2F>(mode, comp, pl, (const Rec2F *)P, nP, (const Rec2F *)Q, nQ, parts, ps.t, c->stream);
+      launch_near<Rec2F>(c, mode, comp, pl, st, ps, parts);
   }
   timer.stop();
   DUGMA_HIP(hipGetLastError());
@@ -658,12 +963,8 @@ static int pose_pass(dugma_ctx *c, const double *R, const double *t, bool iso,
     hipLaunchKernelGGL(k_reduce_parts, dim3(groups), dim3(kBlock), 0, c->stream, parts, (int)nparts, c->dres);
   }
   DUGMA_HIP(hipGetLastError());
-  if (host_sum) {
-    DUGMA_HIP(hipStreamSynchronize(c->stream));
-  } else {
-    rc = wait_slots(c, c->hres, kPosePart * groups);
-    if (rc) return rc;
-  }
+  rc = host_sum ? wait_slots(c, c->hparts, (int)(kPosePart * nparts)) : wait_slots(c, c->hres, kPosePart * groups);
+  if (rc) return rc;
   timer.finish();
   double sum[kPosePart] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (host_sum) {
@@ -696,40 +997,51 @@ static int pose_hess_pass(dugma_ctx *c, const double *R, const double *t, bool i
   if (c->nT == 0 || c->nS == 0) return DUGMA_OK;
   PoseArg ps = make_pose(c, R, t);
   const Plan pl = ctx_plan(c, c->nS, c->nT, kModePose, iso);
-  const size_t nparts = (size_t)pl.pblocks * pl.qchunks;
-  const int groups = (int)std::min<size_t>(kHessGroups, (nparts + kBlock - 1) / kBlock);
-  int rc = c->part.ensure(nparts * kHessPart * sizeof(double));
-  if (!rc) rc = c->scratch2.ensure(sizeof(double) * kHessPart * groups);
-  if (!rc) rc = c->hstage.ensure(sizeof(double) * kHessPart * groups);
-  if (!rc) rc = transform_sources(c, ps, iso);
+  const size_t nparts = (size_t)pl.pblocks * pl.qsplit;
+  const int groups = (int)std::min<size_t>(kRedGroups, (nparts + kBlock - 1) / kBlock);
+  const int tiles = pl.tiles_p * pl.qchunks, hgroups = std::min(tiles, kHessGroups);
+  // scratch: pose partials | tile sums | per chunk and point the Hessian's inputs
+  auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t o_tile = al(nparts * kPosePart * sizeof(double));
+  const size_t o_rec = o_tile + al((size_t)hgroups * kHessPart * sizeof(double));
+  int rc = c->part.ensure(o_rec + (size_t)pl.qchunks * c->nS * kHessRec * sizeof(float));
   if (rc) return rc;
-  double *parts = (double *)c->part.ptr, *gres = (double *)c->scratch2.ptr;
+  char *base = (char *)c->part.ptr;
+  double *parts = (double *)base, *tsum = (double *)(base + o_tile);
+  float *rec = (float *)(base + o_rec);
+  double *hslots = c->hres + dugma_ctx::kResMoments;
+  preset_slots(c->hres, kPosePart * groups);
+  preset_slots(hslots, 21);
   PairTimer timer(c);
+  const Sets st = {1, nullptr, iso ? c->dTrecI : c->dTrecF, pose_lam_scale(3, R)};
   if (iso)
-    launch_pairs_c<Rec3I, kModeHess, 2>(pl, (const Rec3I *)c->dSrecI, c->nS, (const Rec3I *)c->dTrecI, c->nT,
-                                          parts, ps.t, c->stream);
+    launch_near_x<Rec3I, kModeHess, 2, true>(c, pl, st, ps, parts, rec);
   else
-    launch_pairs_c<Rec3F, kModeHess, 2>(pl, (const Rec3F *)c->dSrecF, c->nS, (const Rec3F *)c->dTrecF, c->nT,
-                                          parts, ps.t, c->stream);
+    launch_near_x<Rec3F, kModeHess, 2, true>(c, pl, st, ps, parts, rec);
   timer.stop();
-  hipLaunchKernelGGL(k_reduce_hess, dim3(groups), dim3(kBlock), 0, c->stream, parts, (int)nparts, gres);
+  hipLaunchKernelGGL(k_reduce_parts, dim3(groups), dim3(kBlock), 0, c->stream, parts, (int)nparts, c->dres);
+  hipLaunchKernelGGL(k_hess_tiles, dim3(hgroups), dim3(kBlock), 0, c->stream, rec, c->nS, pl.T, pl.tiles_p, tiles,
+                     tsum);
+  hipLaunchKernelGGL(k_reduce_hess, dim3(1), dim3(1024), 0, c->stream, tsum, hgroups,
+                     c->dres + dugma_ctx::kResMoments);
   DUGMA_HIP(hipGetLastError());
-  DUGMA_HIP(hipMemcpyAsync(c->hstage.ptr, gres, sizeof(double) * kHessPart * groups, hipMemcpyDeviceToHost,
-                           c->stream));
-  DUGMA_HIP(hipStreamSynchronize(c->stream));
+  rc = wait_slots(c, hslots, 21);
+  if (!rc) rc = wait_slots(c, c->hres, kPosePart * groups);
+  if (rc) return rc;
   timer.finish();
-  double sum[kHessUsed];
-  for (int a = 0; a < kHessUsed; ++a) sum[a] = 0.0;
-  const double *hs = (const double *)c->hstage.ptr;
+  double sum[kPosePart], hsum[21];
+  const volatile double *hr = c->hres, *hh = hslots;
+  for (int a = 0; a < kPosePart; ++a) sum[a] = 0.0;
   for (int g = 0; g < groups; ++g)
-    for (int a = 0; a < kHessUsed; ++a) sum[a] += hs[kHessPart * g + a];
+    for (int a = 0; a < kPosePart; ++a) sum[a] += hr[kPosePart * g + a];
+  for (int a = 0; a < 21; ++a) hsum[a] = hh[a];
   // unscale: E ~ s^3, and a factor s per translation index
   const double cn = gauss_norm(3), sc = c->scale, sD = sc * sc * sc;
   res[0] = cn * sD * sum[0];
   for (int a = 1; a < 7; ++a) res[a] = cn * sD * sum[a] * (a > 3 ? sc : 1.0);
   int q = 0;
   for (int i = 0; i < 6; ++i)
-    for (int j = i; j < 6; ++j, ++q) H[q] = cn * sD * sum[kPosePart + q] * (i >= 3 ? sc : 1.0) * (j >= 3 ? sc : 1.0);
+    for (int j = i; j < 6; ++j, ++q) H[q] = cn * sD * hsum[q] * (i >= 3 ? sc : 1.0) * (j >= 3 ? sc : 1.0);
   return DUGMA_OK;
 }
 
@@ -780,36 +1092,37 @@ static void perturb(int D, const double *R, const double *t, const double *p,
 
 constexpr size_t kHostChunk = 4096;  // points per host task of the per-point conversion
 
-// One per-point pass (stationary set P, streamed set Q), full covariance
-// records; writes per-point FP64 sums [nP][NACC] to out (device).
-// Launch: 65,536 waves, at most 64 streamed chunks and 1 GiB of per-chunk
-// partials.  At 76,800 x 76,800 the two passes take 14.9 ms at 55 chunks
-// against 17.6 ms at 7 chunks (8,192 waves).
+// One per-point pass (stationary cloud st.stat), full covariance records;
+// writes per-point FP64 sums [nP][NACC] to out (device).
+// Sub-tiles: chunks for 65,536 waves, at most 64 and 1 GiB of per-chunk sums.
 constexpr size_t kPointPartBytes = size_t(1) << 30;
-static int point_pass(dugma_ctx *c, const void *P, int nP, const void *Q,
-                      int nQ, int comp, double *out) {
+static int point_pass(dugma_ctx *c, const Sets &st, const PoseArg &ps, int comp, double *out) {
   const int D = c->D;
   const int nacc = D == 3 ? kAcc3F : kAcc2F;
+  const int nP = st.stat == 0 ? c->nT : c->nS, nQ = st.stat == 0 ? c->nS : c->nT;
   const int max_chunks =
       (int)std::max<size_t>(1, std::min<size_t>(64, kPointPartBytes / ((size_t)nP * nacc * sizeof(double))));
-  Plan pl = make_plan(nP, nQ, kModePoint, 1, env_int("DUGMA_POINT_WAVES", 65536), max_chunks);
-  const size_t nparts = (size_t)pl.qchunks * nP * nacc;
-  int rc = c->part.ensure(nparts * sizeof(double));
-  if (rc) return rc;
-  double *parts = (double *)c->part.ptr;
-  const double t0[3] = {0, 0, 0};
+  Plan pl = make_plan(nP, nQ, kModePoint, 1, env_int("DUGMA_POINT_WAVES", 65536), kLaunchWaves, max_chunks);
+  double *parts = out;  // one part: the sums themselves
+  if (pl.qsplit > 1) {
+    int rc = c->part.ensure((size_t)pl.qsplit * nP * nacc * sizeof(double));
+    if (rc) return rc;
+    parts = (double *)c->part.ptr;
+  }
   if (!comp_enabled()) comp = 0;
   PairTimer timer(c);
   if (D == 3)
-    launch_pairs<Rec3F>(kModePoint, comp, pl, (const Rec3F *)P, nP, (const Rec3F *)Q, nQ, parts, t0, c->stream);
+    launch_near<Rec3F>(c, kModePoint, comp, pl, st, ps, parts);
   else
-    launch_pairs<Rec2F>(kModePoint, comp, pl, (const Rec2F *)P, nP, (const Rec2F *)Q, nQ, parts, t0, c->stream);
+    launch_near<Rec2F>(c, kModePoint, comp, pl, st, ps, parts);
   timer.stop();
   DUGMA_HIP(hipGetLastError());
-  const size_t total = (size_t)nP * nacc;
-  hipLaunchKernelGGL(k_reduce_points, dim3((unsigned)((total + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->stream,
-                     parts, nP, pl.qchunks, nacc, out);
-  DUGMA_HIP(hipGetLastError());
+  if (pl.qsplit > 1) {
+    const size_t total = (size_t)nP * nacc;
+    hipLaunchKernelGGL(k_reduce_points, dim3((unsigned)((total + kBlock - 1) / kBlock)), dim3(kBlock), 0, c->stream,
+                       parts, nP, pl.qsplit, nacc, out);
+    DUGMA_HIP(hipGetLastError());
+  }
   timer.finish();
   return DUGMA_OK;
 }
@@ -985,8 +1298,10 @@ extern "C" int dugma_energy_grad_points(dugma_ctx *ctx, const double *R,
 
   // per-point passes use full-covariance records (isotropic points included)
   PoseArg ps = make_pose(c, R, t);
-  rc = transform_sources(c, ps, false);
+  const float lam_scale = pose_lam_scale(D, R);
+  rc = transform_sources(c, ps, false, lam_scale);
   if (rc) return rc;
+  const Sets onT = {0, c->dTrecF, c->dSrecF, lam_scale}, onS = {1, c->dSrecF, c->dTrecF, lam_scale};
   const size_t nT = c->nT, nS = c->nS;
   rc = c->scratch2.ensure(sizeof(double) * (nT + nS) * nacc);
   if (rc) return rc;
@@ -999,11 +1314,11 @@ extern "C" int dugma_energy_grad_points(dugma_ctx *ctx, const double *R,
   if (!c->evpts) DUGMA_HIP(hipEventCreateWithFlags(&c->evpts, hipEventDisableTiming));
   // target pass, its sums on their way to the host, then the source pass:
   // the host converts the target sums while the source pass runs
-  rc = point_pass(c, c->dTrecF, c->nT, c->dSrecF, c->nS, 1, acc);
+  rc = point_pass(c, onT, ps, 1, acc);
   hipError_t e = hipSuccess;
   if (!rc) e = hipMemcpyAsync(c->hstage.ptr, acc, sizeof(double) * nT * nacc, hipMemcpyDeviceToHost, c->stream);
   if (!rc && e == hipSuccess) e = hipEventRecord(c->evpts, c->stream);
-  if (!rc && e == hipSuccess) rc = point_pass(c, c->dSrecF, c->nS, c->dTrecF, c->nT, 2, acc + nT * nacc);
+  if (!rc && e == hipSuccess) rc = point_pass(c, onS, ps, 2, acc + nT * nacc);
   if (!rc && e == hipSuccess)
     e = hipMemcpyAsync((double *)c->hstage.ptr + nT * nacc, acc + nT * nacc, sizeof(double) * nS * nacc,
                        hipMemcpyDeviceToHost, c->stream);
@@ -1191,12 +1506,7 @@ extern "C" int dugma_autotune(dugma_ctx *ctx, int cov_mode) {
   hipEvent_t e0, e1;
   DUGMA_HIP(hipEventCreate(&e0));
   DUGMA_HIP(hipEventCreate(&e1));
-  static const int kT[2] = {1, 2};
-  // The largest targets serve large problems: at 200K x 200K the kernel
-  // takes 17.75 ms at 32,768 waves (11 source chunks), 16.89 ms at 131,072
-  // (42) and 16.70-16.76 ms at 524,288 (168).
-  static const int kW[] = {2048, 4096, 8192, 16384, 32768, 65536, 131072, 262144, 524288};
-  constexpr int kNW = (int)(sizeof(kW) / sizeof(kW[0]));
+  static const int kW[] = {2048, 4096, 8192, 16384, 32768};
   const double pairs = (double)ctx->nT * ctx->nS;
   const int reps = pairs > 4e9 ? 1 : (pairs > 1e8 ? 3 : 10);
   for (int m = 0; m < 2; ++m) {
@@ -1205,29 +1515,27 @@ extern "C" int dugma_autotune(dugma_ctx *ctx, int cov_mode) {
     float best_ms = 1e30f;
     // the stationary and streamed sets of pose_pass
     const int nP = sources_stationary() ? ctx->nS : ctx->nT, nQ = sources_stationary() ? ctx->nT : ctx->nS;
-    for (int ti = 0; ti < 2; ++ti) {
-      int last_chunks = -1;
-      for (int wi = 0; wi < kNW; ++wi) {
-        // targets that give the launch of the previous one are not timed again
-        const int chunks = make_plan(nP, nQ, mode, kT[ti], kW[wi]).qchunks;
-        if (chunks == last_chunks) continue;
-        last_chunks = chunks;
-        dugma_ctx::Tuned &tu = ctx->tuned[m][iso ? 1 : 0];
-        tu.T = kT[ti];
-        tu.target_waves = kW[wi];
-        double res[kPosePart];
-        rc = pose_pass(ctx, R, t, iso, mode, res);  // warm
-        if (rc) break;
-        (void)hipEventRecord(e0, ctx->stream);
-        for (int r = 0; r < reps && !rc; ++r) rc = pose_pass(ctx, R, t, iso, mode, res);
-        (void)hipEventRecord(e1, ctx->stream);
-        (void)hipEventSynchronize(e1);
-        float ms = 0.0f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
-        if (!rc && ms < best_ms) {
-          best_ms = ms;
-          best = tu;
-        }
+    int last_split = -1;
+    for (const int waves : kW) {
+      dugma_ctx::Tuned &tu = ctx->tuned[m][iso ? 1 : 0];
+      tu.T = 1;
+      tu.target_waves = waves;
+      // targets that give the launch of the previous one are not timed again
+      const int split = ctx_plan(ctx, nP, nQ, mode, iso).qsplit;
+      if (split == last_split) continue;
+      last_split = split;
+      double res[kPosePart];
+      rc = pose_pass(ctx, R, t, iso, mode, res);  // warm
+      if (rc) break;
+      (void)hipEventRecord(e0, ctx->stream);
+      for (int r = 0; r < reps && !rc; ++r) rc = pose_pass(ctx, R, t, iso, mode, res);
+      (void)hipEventRecord(e1, ctx->stream);
+      (void)hipEventSynchronize(e1);
+      float ms = 0.0f;
+      (void)hipEventElapsedTime(&ms, e0, e1);
+      if (!rc && ms < best_ms) {
+        best_ms = ms;
+        best = tu;
       }
     }
     ctx->tuned[m][iso ? 1 : 0] = best;

@@ -172,6 +172,17 @@ struct PinBuf {
   void release();
 };
 
+// One cloud's spatial index (dugma_near.h): its n kept points in Hilbert
+// order.
+struct QAux;
+struct QBox;
+struct NearCloud {
+  int *ord = nullptr;    // Hilbert position -> kept index
+  QAux *aux = nullptr;   // by Hilbert position: FP32 position and lam
+  QBox *box = nullptr;   // per 64 Hilbert positions
+  float *lam = nullptr;  // by Hilbert position: bound of the covariance's largest eigenvalue
+};
+
 }  // namespace dugma
 
 struct dugma_ctx;
@@ -230,7 +241,7 @@ struct dugma_ctx {
 
   // launch shapes chosen by dugma_autotune: [energy / pose][full / iso]
   struct Tuned {
-    int T = 2;
+    int T = 1;             // stationary points per lane
     int target_waves = 0;  // 0: not tuned
   };
   Tuned tuned[2][2];
@@ -241,6 +252,9 @@ struct dugma_ctx {
   hipEvent_t evpts = nullptr;  // per-point gradients: the target sums have reached the host
   double pair_ms = 0.0;
   long long pair_launches = 0;
+
+  dugma::NearCloud near[2];  // spatial index: targets, sources
+  dugma::DevBuf nearbuf;     // its arrays
 
   dugma::DevBuf part;        // pair-kernel partials
   dugma::DevBuf scratch2;    // reductions / k-NN merge

@@ -14,6 +14,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "dugma_internal.h"
+#include "dugma_near.h"
 #include "dugma_pairs.h"
 
 namespace dugma {
@@ -1161,6 +1162,8 @@ extern "C" int dugma_update_sigma_knn(dugma_ctx *ctx, int which, int k, float *s
     }
 #undef SIGMA_APPLY
     DUGMA_HIP(hipGetLastError());
+    rc = near_refresh(c, cloud);
+    if (rc) return rc;
   }
   // counts (and the sigmas, when asked for) back to the host
   const bool wantT = sigma_target && doT, wantS = sigma_source && doS;
@@ -1261,6 +1264,8 @@ extern "C" int dugma_update_cov_knn(dugma_ctx *ctx, int which, int k, double sca
     }
 #undef COV_APPLY
     DUGMA_HIP(hipGetLastError());
+    rc = near_refresh(c, cloud);
+    if (rc) return rc;
   }
   const bool wantT = sigma_target && doT, wantS = sigma_source && doS;
   const size_t hbytes = 16 + (wantT ? (size_t)nT * 4 : 0) + (wantS ? (size_t)nS * 4 : 0);
