@@ -20,16 +20,16 @@
 // calls update_sig before its loop.  Optionally an extra variance a -> 0 is
 // annealed on top.
 //
-// One iteration for all trials is four kernels:
-//   k_batch_transform  the targets in each trial's source frame,
-//                      z_i = R_k^T (y_i - (t_k - c_k)) (FP64, rounded to
-//                      FP32), and g s_i + a; the sources stay as given (FP32)
-//   k_batch_pairs      persistent; workgroups pop (trial, target tile, source
-//                      chunk) items from a queue ordered longest first and
-//                      write FP64 sufficient statistics per item, plus the
+// One iteration for all trials is three kernels:
+//   k_batch_pairs      persistent; workgroups pop units from a queue ordered
+//                      longest first -- 64 targets of a (trial, target tile,
+//                      source chunk) item -- take the targets to the trial's
+//                      source frame, z_i = R_k^T (y_i - (t_k - c_k)) (FP64,
+//                      rounded to FP32; the sources stay as given), and
+//                      write the unit's FP64 sufficient statistics, plus the
 //                      per-target nearest squared distance
 //   k_batch_fold       one workgroup per trial: its nearest-distance sum
-//                      and a fixed-order sum of its items; re-arms the queue
+//                      and a fixed-order sum of its units; re-arms the queue
 //   k_batch_update     one thread per trial: Horn's quaternion solution
 //                      (4x4 Jacobi, FP64), pose, sigma, annealing,
 //                      convergence
@@ -49,14 +49,14 @@
 // neighbours -- make the energy's maximum sit at the true pose) by BFGS on
 // -log E over left pose increments, one fused energy + pose-gradient pass per
 // trial pose (the logic of dugma_register_energy, one thread per trial):
-//   k_batchf_transform  targets and their covariances in each trial's source
-//                       frame at the candidate pose (FP64 -> FP32 hi/lo)
-//   k_batchf_pairs      the same persistent item queue; per target lane E,
-//                       EW and B (full covariance), then the pose gradient
+//   k_batchf_pairs      the same persistent queue of units; the targets and
+//                       their covariances in the trial's source frame at the
+//                       candidate pose (FP64 -> FP32 hi/lo), per target lane
+//                       E, EW and B (full covariance), then the pose gradient
 //                       by the target-side identity, in the source frame;
-//                       a wave skips each block of 64 sources whose terms
+//                       a unit skips each block of 64 sources whose terms
 //                       are all below 7e-13 of their peaks (kFarExp)
-//   k_batchf_fold       sums each running trial's items (one workgroup each)
+//   k_batchf_fold       sums each running trial's units (one workgroup each)
 //   k_batchf_update     one thread per trial: rotates the gradient back, Armijo
 //                       test, BFGS update, next candidate pose; at an
 //                       accepted pose the direction comes from the pass's
@@ -73,10 +73,12 @@
 // sparser levels are then evenly spread subsamples, and 64 consecutive
 // points lie close together, which the far-field skip needs.
 //
-// Launch shape: waves per workgroup (target tile = 64 x waves), the number
-// of source chunks per target tile for each size class of trials (by source
+// Launch shape: 64-target units per target tile ("waves"), the number of
+// source chunks per target tile for each size class of trials (by source
 // count), and the resident waves of the persistent kernel are chosen by
 // dugma_batch_autotune, which times whole iterations on the batch's own data.
+// Tiles and chunks say how the FP64 sums are grouped; how many waves share a
+// unit's sources (iso_waves) does not change a result.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -85,6 +87,7 @@
 #include <vector>
 
 #include "dugma_internal.h"
+#include "dugma_near.h"
 #include "dugma_pairs.h"
 
 namespace dugma {
@@ -92,6 +95,7 @@ namespace dugma {
 constexpr int kBSub = 64;
 constexpr int kStat = 28;         // stride of the per-item statistics (doubles; 17 / 28 used)
 constexpr int kUpd = 256;         // threads of the fold kernel (one workgroup per trial)
+constexpr int kUpdItems = 64;     // items it stages at a time
 constexpr int kClasses = 4;       // size classes by source count: < 1000, < 2000, < 4000, more
 constexpr unsigned kInfBits = 0x7f800000u;  // +inf as u32: start value of the nearest distance
 constexpr double kGMin = 1e-6;    // smallest variance scale g
@@ -103,9 +107,11 @@ static inline int size_class(int ns) { return ns < 1000 ? 0 : ns < 2000 ? 1 : ns
 
 // A work item: targets [t0, t0 + tn) of a trial against its sources
 // [s0, s0 + sn); s0 sits a multiple of 64 sources into the trial's, and blk
-// is the index of its first 64-source block in the level's block bounds.
+// is the index of its first 64-source block in the level's block bounds.  Its
+// units are the tile's 64-target pieces: nu of them, with statistics records
+// u0, u0 + 1, ... (u0: the item times the tile's size in units); a queue entry is 4 item + piece (a tile has at most 4).
 struct BItem {
-  int trial, t0, tn, s0, sn, blk, pad1, pad2;
+  int trial, t0, tn, s0, sn, blk, u0, nu;
 };
 
 struct BTrial {
@@ -142,27 +148,17 @@ struct alignas(16) BSrc {
 
 // A target in its trial's source frame at the current pose: z (FP32),
 // s = (g s_i + a) ln 4 and the trial's variance scale g.
-struct alignas(16) BZ {
-  float x, y, z, s, g, pad0, pad1, pad2;
+struct BZ {
+  float x, y, z, s, g;
 };
 
-// Per iteration, for every target of a running trial: z = R^T (y - (t - c))
-// in FP64 (y relative to the trial's target centroid c), rounded to FP32,
-// with (g s_i + a) ln 4 and g.  z - x_j = R^T (y - R x_j - t) has the
-// length of the pair difference in the target frame.  Rounding z moves the
-// target by at most half an FP32 ulp of its coordinates (~3e-8 of the
-// trial's extent), a millionth of the kernel width at the smallest sigma
+// z = R^T (y - (t - c)) in FP64 (y relative to the trial's target centroid c),
+// rounded to FP32, with (g s_i + a) ln 4 and g.  z - x_j = R^T (y - R x_j - t)
+// has the length of the pair difference in the target frame.  Rounding z
+// moves the target by at most half an FP32 ulp of its coordinates (~3e-8 of
+// the trial's extent), a millionth of the kernel width at the smallest sigma
 // the trials have.
-__global__ __launch_bounds__(256) void k_batch_transform(
-    const Rec3I *__restrict__ T, const int *__restrict__ tgt_trial, int i0,
-    int i1, const BTrial *__restrict__ trials, const int *__restrict__ done,
-    BZ *__restrict__ Z) {
-  const int i = i0 + blockIdx.x * 256 + threadIdx.x;
-  if (i >= i1) return;
-  const int k = tgt_trial[i];
-  if (done[k]) return;
-  const BTrial &tr = trials[k];
-  const Rec3I y = T[i];
+__device__ __forceinline__ BZ batch_target(const Rec3I &y, const BTrial &tr) {
   const double u[3] = {(double)y.hx - (tr.t[0] - tr.c[0]), (double)y.hy - (tr.t[1] - tr.c[1]),
                        (double)y.hz - (tr.t[2] - tr.c[2])};
   double v[3];
@@ -179,8 +175,7 @@ __global__ __launch_bounds__(256) void k_batch_transform(
   r.z = (float)v[2];
   r.s = (float)fma(tr.g, (double)y.s, tr.a * kLn4);  // y.s holds s_i ln 4
   r.g = (float)tr.g;
-  r.pad0 = r.pad1 = r.pad2 = 0.0f;
-  Z[i] = r;
+  return r;
 }
 
 __global__ __launch_bounds__(256) void k_batch_fill(unsigned *__restrict__ p, int n, unsigned v) {
@@ -215,102 +210,250 @@ __global__ __launch_bounds__(256) void k_batch_resig(BTrial *__restrict__ trials
 //    of E.
 // With SIG the item's smallest |d_ij|^2 per target is folded into nn[i]
 // (atomicMin on the bits of a non-negative float, which order like the
-// values).  The source stream is software-pipelined two deep: record j + 2
-// is requested while record j is used (index clamped to the item), so the
-// scalar-load latency overlaps the arithmetic.
+// values).
 // EN: also sum E_i.  The pose step does not need it, so the iterations
 // leave it out (one VALU operation per pair fewer) and one pass with EN
 // after the iterations measures the energy at the returned poses.
+//
+// A workgroup's S waves hold the same 64 targets and share the unit's blocks
+// of 64 sources, S at a time: each wave sums one block in FP32 (its sources
+// staged in LDS and read back one by one at a wave-uniform address, so that
+// every operand of a pair is a VGPR), leaves the sums in LDS, and after a
+// barrier the sums' owners (sum a: wave a mod S) add the S blocks' to their
+// FP64 sums in block order -- the order one wave alone would have added them
+// in, so S changes no result.  With one wave per 64 targets, 64 trials of 500 to
+// 8,000 points (731 units) were bound by the latency of that wave's chain of
+// pairs, the chip nearly idle: 168 us per coarse pass, 42 with the blocks shared
+// (12.5K VALU quad-cycles per SIMD; the longest units' CUs finish last).
 constexpr int kItemStat = 17;
-template <int W, bool SIG, bool EN>
-__global__ __launch_bounds__(64 * W) void k_batch_pairs(
-    const Rec3I *__restrict__ T, const BZ *__restrict__ Z, const BSrc *__restrict__ S,
-    const BItem *__restrict__ items, const int *__restrict__ order, int nitems,
+
+// The units of a workgroup: its own index first, then, where the grid is smaller
+// than the queue, the next one not taken yet -- asked for at the start of a unit
+// and published (LDS) at its end, so that the answer's latency lies under the
+// unit's work.  (Atomics of all workgroups on the one counter are served one
+// after another: as the first unit's source they cost 64 trials 2.5 ms of a
+// registration's 20.)  The barrier follows the write directly: at the head of the unit
+// loop, ROCm 7.2's hipcc drops the wait for the write from it.
+struct UnitQueue {
+  unsigned *queue;
+  int *slot;  // two LDS entries
+  int turn = 0, next = 0;
+  bool first = true;
+  __device__ UnitQueue(unsigned *q, int *s) : queue(q), slot(s) {}
+  __device__ int take(int nunits) {
+    const int p = first ? (int)blockIdx.x : __builtin_amdgcn_readfirstlane(slot[turn]);
+    if ((int)gridDim.x < nunits && p < nunits && threadIdx.x == 0) next = (int)(gridDim.x + atomicAdd(queue, 1u));
+    return p;
+  }
+  // after every wave is done with the last unit's LDS
+  __device__ void publish(int nunits) {
+    first = false;
+    turn ^= 1;
+    if (threadIdx.x == 0) slot[turn] = (int)gridDim.x < nunits ? next : nunits;
+    __syncthreads();
+  }
+};
+
+// Orders a wave's own LDS writes and reads (no other wave uses them).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One round of a unit: each wave's FP32 block sums (where it had a block: nb
+// waves) through LDS to their owners, who add them in block order.
+template <int S, int NA>
+__device__ __forceinline__ void add_blocks(float *x, const float *acc, bool has, int nb, int wave, int lane,
+                                           double *d) {
+  if (has) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a) x[(wave * NA + a) * 64 + lane] = acc[a];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i * S < NA; ++i) {
+    const int a = wave + i * S;
+    if (a < NA) {
+      if (nb == S) {
+#pragma unroll
+        for (int k = 0; k < S; ++k) d[i] += (double)x[(k * NA + a) * 64 + lane];
+      } else {
+        for (int k = 0; k < nb; ++k) d[i] += (double)x[(k * NA + a) * 64 + lane];
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// The owners' FP64 sums to every wave.
+template <int S, int NA>
+__device__ __forceinline__ void share_sums(const double *d, double *tot, int wave, int lane, double *all) {
+#pragma unroll
+  for (int i = 0; i * S < NA; ++i)
+    if (wave + i * S < NA) tot[(wave + i * S) * 64 + lane] = d[i];
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < NA; ++a) all[a] = tot[a * 64 + lane];
+}
+
+// One pair: a lane's target and a source read from LDS.  acc: [W, D (3), E].
+template <bool SIG, bool EN>
+__device__ __forceinline__ void iso_pair(const BZ &z, const float4 q, float *acc, float &dmin) {
+  const float dx = z.x - q.x;
+  const float dy = z.y - q.y;
+  const float dz = z.z - q.z;
+  const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+  if (SIG) dmin = fminf(dmin, d2);
+  const float rs = frsq(fmaf(q.w, z.g, z.s));
+  const float inv = rs * rs;
+  const float e = fexp2(-(d2 * inv)) * (rs * inv);
+  const float w = e * inv;
+  acc[0] += w;
+  acc[1] = fmaf(w, dx, acc[1]);
+  acc[2] = fmaf(w, dy, acc[2]);
+  acc[3] = fmaf(w, dz, acc[3]);
+  if (EN) acc[4] += e;
+}
+
+// A unit's totals, one statistic at a time, dealt to its S waves: [E, W,
+// W y (3), B' (3), y B'^T (9)].  sum: the lane's W, D (3), E.
+template <int S, bool EN>
+__device__ __forceinline__ void unit_totals(const Rec3I &pt, const BZ &pz, const double *sum, bool valid, int wave,
+                                            int lane, double *__restrict__ o) {
+  const double dW = sum[0];
+  const double y[3] = {(double)pt.hx, (double)pt.hy, (double)pt.hz};
+  const double z[3] = {(double)pz.x, (double)pz.y, (double)pz.z};
+  const double dB[3] = {fma(dW, z[0], -sum[1]), fma(dW, z[1], -sum[2]), fma(dW, z[2], -sum[3])};
+#pragma unroll
+  for (int a = 0; a < kItemStat; ++a) {
+    if (a % S != wave) continue;  // uniform
+    double v;
+    if (a == 0)
+      v = EN ? sum[4] : 0.0;
+    else if (a == 1)
+      v = dW;
+    else if (a < 5)
+      v = dW * y[a - 2];
+    else if (a < 8)
+      v = dB[a - 5];
+    else
+      v = y[(a - 8) / 3] * dB[(a - 8) % 3];
+    v = wave_sum(valid ? v : 0.0);
+    if (lane == 0) o[a] = v;
+  }
+}
+
+template <int S, bool SIG, bool EN>
+__global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_batch_pairs(
+    const Rec3I *__restrict__ T, const BTrial *__restrict__ trials, const BSrc *__restrict__ Sr,
+    const BItem *__restrict__ items, const int *__restrict__ order, int nunits,
     unsigned *__restrict__ queue, const int *__restrict__ done,
     unsigned *__restrict__ nn, double *__restrict__ part) {
-  __shared__ int s_p;
-  __shared__ double red[W][kItemStat];
+  constexpr int NA = EN ? 5 : 4;
+  __shared__ int s_slot[2];
+  __shared__ float4 s_src[S][64];
+  __shared__ float s_x[S * NA * 64];
+  __shared__ double s_tot[NA * 64];
+  __shared__ float s_min[SIG ? S * 64 : 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (;;) {
-    if (threadIdx.x == 0) s_p = (int)atomicAdd(queue, 1u);
-    __syncthreads();
-    const int p = __builtin_amdgcn_readfirstlane(s_p);
-    __syncthreads();
-    if (p >= nitems) break;
-    const int idx = __builtin_amdgcn_readfirstlane(order[p]);
-    const BItem it = items[idx];
+  UnitQueue uq(queue, s_slot);
+  for (int p; (p = uq.take(nunits)) < nunits; uq.publish(nunits)) {
+    const int code = __builtin_amdgcn_readfirstlane(order[p]), u = code & 3;
+    const BItem it = items[code >> 2];
     if (done[it.trial]) continue;
-    const int ti = it.t0 + wave * 64 + lane;
-    const bool valid = (wave * 64 + lane) < it.tn;
-    const BZ pz = Z[valid ? ti : it.t0];
-    const float g = pz.g, cs = pz.s;
-    double dE = 0.0, dW = 0.0, dD[3] = {0.0, 0.0, 0.0};
+    const bool valid = u * 64 + lane < it.tn;
+    const int ti = valid ? it.t0 + u * 64 + lane : it.t0;
+    const Rec3I pt = T[ti];
+    const BZ pz = batch_target(pt, trials[it.trial]);
+    const int nblk = (it.sn + kBSub - 1) / kBSub;
+    double d[(NA + S - 1) / S];
+#pragma unroll
+    for (int i = 0; i * S < NA; ++i) d[i] = 0.0;
+    float dmin = __builtin_huge_valf();
+    const float4 *src = reinterpret_cast<const float4 *>(Sr + it.s0);
+    float4 own = src[min(wave * kBSub + lane, it.sn - 1)];
+    for (int b0 = 0; b0 < nblk; b0 += S) {
+      const int b = b0 + wave;
+      float acc[NA];
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
+      if (b < nblk) {
+        const int n = min(kBSub, it.sn - b * kBSub);
+        s_src[wave][lane] = own;
+        own = src[min((b + S) * kBSub + lane, it.sn - 1)];  // the wave's next block
+        wave_lds_fence();
+        int j = 0;
+        for (; j + 8 <= n; j += 8) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) iso_pair<SIG, EN>(pz, s_src[wave][j + k], acc, dmin);
+        }
+        for (; j < n; ++j) iso_pair<SIG, EN>(pz, s_src[wave][j], acc, dmin);
+        wave_lds_fence();
+      }
+      add_blocks<S, NA>(s_x, acc, b < nblk, min(S, nblk - b0), wave, lane, d);
+    }
+    if (SIG) s_min[wave * 64 + lane] = dmin;
+    double sum[NA];  // W, D (3), E
+    share_sums<S, NA>(d, s_tot, wave, lane, sum);
+    if (SIG && wave == 0) {
+#pragma unroll
+      for (int k = 1; k < S; ++k) dmin = fminf(dmin, s_min[k * 64 + lane]);
+      if (valid) atomicMin(nn + ti, __float_as_uint(dmin));
+    }
+    unit_totals<S, EN>(pt, pz, sum, valid, wave, lane, part + (size_t)(it.u0 + u) * kStat);
+  }
+}
+
+// The same where the units alone fill the chip (iso_waves): each of a
+// workgroup's 4 waves takes a unit of its own, 4 neighbours in the queue, so
+// mostly of one item with the same sources, and streams them through SGPRs,
+// record j + 2 requested while record j is used (index clamped to the chunk).
+// 2,048 trials, 12 iterations on the full clouds without the sigma update:
+// 70 ms, with shared blocks 79 (their LDS reads).
+constexpr int kWideUnits = 4;
+template <bool SIG, bool EN>
+__global__ __launch_bounds__(64 * kWideUnits) void k_batch_pairs_wide(
+    const Rec3I *__restrict__ T, const BTrial *__restrict__ trials, const BSrc *__restrict__ Sr,
+    const BItem *__restrict__ items, const int *__restrict__ order, int nunits,
+    unsigned *__restrict__ queue, const int *__restrict__ done,
+    unsigned *__restrict__ nn, double *__restrict__ part) {
+  constexpr int NA = EN ? 5 : 4;
+  __shared__ int s_slot[2];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ngroups = (nunits + kWideUnits - 1) / kWideUnits;
+  UnitQueue uq(queue, s_slot);
+  for (int p; (p = uq.take(ngroups)) < ngroups; uq.publish(ngroups)) {
+    if (p * kWideUnits + wave >= nunits) continue;
+    const int code = __builtin_amdgcn_readfirstlane(order[p * kWideUnits + wave]), u = code & 3;
+    const BItem it = items[code >> 2];
+    if (done[it.trial]) continue;
+    const bool valid = u * 64 + lane < it.tn;
+    const int ti = valid ? it.t0 + u * 64 + lane : it.t0;
+    const Rec3I pt = T[ti];
+    const BZ pz = batch_target(pt, trials[it.trial]);
+    double sum[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) sum[a] = 0.0;
     float dmin = __builtin_huge_valf();
     const int s_end = it.s0 + it.sn;
-    // a wave past the tile's last target skips the pair loop (its sums stay
-    // zero, as its masked lanes would have made them)
-    const int s_run = wave * 64 < it.tn ? s_end : it.s0;
-    BSrc qa = S[it.s0], qb = S[min(it.s0 + 1, s_end - 1)];  // it.sn >= 1
-    for (int j0 = it.s0; j0 < s_run; j0 += kBSub) {
-      float fE = 0.0f, fW = 0.0f, fD0 = 0.0f, fD1 = 0.0f, fD2 = 0.0f;
+    BSrc qa = Sr[it.s0], qb = Sr[min(it.s0 + 1, s_end - 1)];  // it.sn >= 1
+    for (int j0 = it.s0; j0 < s_end; j0 += kBSub) {
+      float acc[NA];
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
       const int j1 = min(j0 + kBSub, s_end);
 #pragma unroll 2
       for (int j = j0; j < j1; ++j) {
         const BSrc q = qa;
         qa = qb;
-        qb = S[min(j + 2, s_end - 1)];
-        const float dx = pz.x - q.x;
-        const float dy = pz.y - q.y;
-        const float dz = pz.z - q.z;
-        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-        if (SIG) dmin = fminf(dmin, d2);
-        const float rs = frsq(fmaf(q.s, g, cs));
-        const float inv = rs * rs;
-        const float e = fexp2(-(d2 * inv)) * (rs * inv);
-        const float w = e * inv;
-        if (EN) fE += e;
-        fW += w;
-        fD0 = fmaf(w, dx, fD0);
-        fD1 = fmaf(w, dy, fD1);
-        fD2 = fmaf(w, dz, fD2);
+        qb = Sr[min(j + 2, s_end - 1)];
+        iso_pair<SIG, EN>(pz, make_float4(q.x, q.y, q.z, q.s), acc, dmin);
       }
-      dE += fE;
-      dW += fW;
-      dD[0] += fD0;
-      dD[1] += fD1;
-      dD[2] += fD2;
+#pragma unroll
+      for (int a = 0; a < NA; ++a) sum[a] += (double)acc[a];
     }
     if (SIG && valid) atomicMin(nn + ti, __float_as_uint(dmin));
-    // item totals, one statistic at a time (few registers live): [E, W,
-    // W y (3), B' (3), y B'^T (9)]
-    const Rec3I pt = T[valid ? ti : it.t0];
-    const double y[3] = {(double)pt.hx, (double)pt.hy, (double)pt.hz};
-    const double z[3] = {(double)pz.x, (double)pz.y, (double)pz.z};
-    const double dB[3] = {fma(dW, z[0], -dD[0]), fma(dW, z[1], -dD[1]), fma(dW, z[2], -dD[2])};
-#pragma unroll
-    for (int a = 0; a < kItemStat; ++a) {
-      double v;
-      if (a == 0)
-        v = dE;
-      else if (a == 1)
-        v = dW;
-      else if (a < 5)
-        v = dW * y[a - 2];
-      else if (a < 8)
-        v = dB[a - 5];
-      else
-        v = y[(a - 8) / 3] * dB[(a - 8) % 3];
-      v = wave_sum(valid ? v : 0.0);
-      if (lane == 0) red[wave][a] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x < kItemStat) {
-      double s = red[0][threadIdx.x];
-#pragma unroll
-      for (int w = 1; w < W; ++w) s += red[w][threadIdx.x];
-      part[(size_t)idx * kStat + threadIdx.x] = s;
-    }
-    __syncthreads();
+    unit_totals<1, EN>(pt, pz, sum, valid, 0, lane, part + (size_t)(it.u0 + u) * kStat);
   }
 }
 
@@ -373,15 +516,41 @@ __device__ void eig4_max(double A[4][4], double q[4]) {
     }
 }
 
+// Statistic a of an item: its W units' in order (a tile's missing units stay 0).
+__device__ __forceinline__ double item_stat(const double *__restrict__ part, int item, int W, int a) {
+  const double *p = part + (size_t)item * W * kStat + a;
+  double v = p[0];
+  if (W >= 2) v += p[kStat];
+  if (W == 4) v = (v + p[2 * kStat]) + p[3 * kStat];
+  return v;
+}
+
+// Items [i0, i1) of a trial, kUpdItems at a time, into LDS; thread a < n then
+// sums statistic a in item order.
+__device__ __forceinline__ double fold_items(const double *__restrict__ part, int i0, int i1, int W, int n,
+                                             double *s_part) {
+  double acc = 0.0;
+  for (int ib = i0; ib < i1; ib += kUpdItems) {
+    const int nb = min(kUpdItems, i1 - ib);
+#pragma unroll 4
+    for (int e = threadIdx.x; e < nb * kStat; e += kUpd)
+      s_part[e] = item_stat(part, ib + e / kStat, W, e % kStat);
+    __syncthreads();
+    if ((int)threadIdx.x < n)
+      for (int i = 0; i < nb; ++i) acc += s_part[i * kStat + threadIdx.x];
+    __syncthreads();
+  }
+  return acc;
+}
+
 // One workgroup per trial.  All threads fold the trial's nearest distances
 // (and reset them for the next pass) into sig = mean / 3 (-1: none), and
 // stage the item statistics in LDS a block of items at a time, from which
 // thread a < 17 sums statistic a in item order.  fold[k] receives the 17
 // sums and, at index 17, sig.
-constexpr int kUpdItems = 64;  // items staged per block
 __global__ __launch_bounds__(kUpd) void k_batch_fold(
-    const double *__restrict__ part, const int *__restrict__ titem, const int *__restrict__ ttgt, int k0,
-    int k1, const BTrial *__restrict__ trials, const int *__restrict__ done, unsigned *__restrict__ queue,
+    const double *__restrict__ part, int W, const int *__restrict__ titem,
+    const int *__restrict__ ttgt, int k0, int k1, const BTrial *__restrict__ trials, const int *__restrict__ done, unsigned *__restrict__ queue,
     unsigned *__restrict__ nn, double *__restrict__ fold, int sigma) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0u;
   const int k = k0 + blockIdx.x;
@@ -408,16 +577,7 @@ __global__ __launch_bounds__(kUpd) void k_batch_fold(
   }
   if (sigma && !trials[k].sig_ready) return;  // this pass only measures sig
   __shared__ double s_part[kUpdItems * kStat];
-  const int i0 = titem[k], i1 = titem[k + 1];
-  double acc = 0.0;
-  for (int ib = i0; ib < i1; ib += kUpdItems) {
-    const int nb = min(kUpdItems, i1 - ib);
-    for (int e = threadIdx.x; e < nb * kStat; e += kUpd) s_part[e] = part[(size_t)ib * kStat + e];
-    __syncthreads();
-    if (threadIdx.x < kItemStat)
-      for (int i = 0; i < nb; ++i) acc += s_part[i * kStat + threadIdx.x];
-    __syncthreads();
-  }
+  const double acc = fold_items(part, titem[k], titem[k + 1], W, kItemStat, s_part);
   if (threadIdx.x < kItemStat) f[threadIdx.x] = acc;
 }
 
@@ -547,13 +707,13 @@ __global__ __launch_bounds__(64) void k_batch_update(const double *__restrict__ 
 // After the isotropic iterations: each trial's energy at its pose, from the
 // item sums of one energy pass (in item order); the queue is re-armed.
 __global__ __launch_bounds__(256) void k_batch_energy(const double *__restrict__ part,
-                                                      const int *__restrict__ titem, int K,
+                                                      int W, const int *__restrict__ titem, int K,
                                                       BTrial *__restrict__ trials, unsigned *__restrict__ queue) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0u;
   const int k = blockIdx.x * 256 + threadIdx.x;
   if (k >= K) return;
   double e = 0.0;
-  for (int i = titem[k]; i < titem[k + 1]; ++i) e += part[(size_t)i * kStat];
+  for (int i = titem[k]; i < titem[k + 1]; ++i) e += item_stat(part, i, W, 0);
   trials[k].E = e * kLn4Pow1p5;  // e was computed with variances times ln 4
 }
 
@@ -608,25 +768,14 @@ struct RParams {
 
 constexpr int kRefStat = 28;  // per refinement item: E, gradient (6), Hessian (21)
 
-// Candidate pose as every pass sees it: z = cR^T (y - (ct - c)) and
-// S' = cR^T S cR, FP64 -> FP32 (position hi + lo).
-__global__ __launch_bounds__(256) void k_batchf_transform(
-    const Rec3I *__restrict__ T, const BCov *__restrict__ TC, const int *__restrict__ tgt_trial, int i0,
-    int i1, const BTrial *__restrict__ trials, const BRef *__restrict__ ref, const int *__restrict__ done,
-    Rec3F *__restrict__ Z) {
-  const int i = i0 + blockIdx.x * 256 + threadIdx.x;
-  if (i >= i1) return;
-  const int k = tgt_trial[i];
-  if (done[k]) return;
-  const BRef &r = ref[k];
-  const double *c = trials[k].c;
-  const Rec3I y = T[i];
+// A target at the candidate pose: z = cR^T (y - (ct - c)) and S' = cR^T S cR,
+// FP64 -> FP32 (position hi + lo).
+__device__ __forceinline__ Rec3F batchf_target(const Rec3I &y, const BCov &cv, const BRef &r, const double *c) {
   const double u[3] = {(double)y.hx - (r.ct[0] - c[0]), (double)y.hy - (r.ct[1] - c[1]),
                        (double)y.hz - (r.ct[2] - c[2])};
   double z[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) z[a] = r.cR[3 * a] * u[0] + r.cR[3 * a + 1] * u[1] + r.cR[3 * a + 2] * u[2];
-  const BCov cv = TC[i];
   const double S[9] = {cv.s11, cv.s12, cv.s13, cv.s12, cv.s22, cv.s23, cv.s13, cv.s23, cv.s33};
   double SR[9], Sp[9];  // S cR, then cR^T S cR (column-major)
 #pragma unroll
@@ -654,26 +803,27 @@ __global__ __launch_bounds__(256) void k_batchf_transform(
   o.s23 = (float)(0.5 * (Sp[7] + Sp[5]));
   o.pad0 = cv.lam;  // the largest eigenvalue does not change with the rotation
   o.pad1 = o.pad2 = o.pad3 = 0.0f;
-  Z[i] = o;
+  return o;
 }
 
-// Per item: the targets of a tile (lanes, hi + lo, in the source frame)
-// against a chunk of sources (static records, streamed two deep through
-// SGPRs): per target E, EW = sum e S^-1 d and B = sum e (S^-1 d d^T S^-1 -
+// Per unit: 64 targets (lanes, hi + lo, in the source frame) against a chunk of
+// sources (static records; the waves share the blocks as in k_batch_pairs): per
+// target E, EW = sum e S^-1 d and B = sum e (S^-1 d d^T S^-1 -
 // S^-1), FP32 over sub-tiles of kBSub sources, then FP64; the pose
 // gradient follows from these target-side sums (pose_contrib: rotation
-// about the origin of the frame, i.e. about t, then translation).  Item
+// about the origin of the frame, i.e. about t, then translation).  Unit
 // totals: [E, rotation (3), translation (3), Hessian (21, pose_hessian_entry,
 // FP32 wave sums)], in the source frame.
+__device__ __forceinline__ float lane_f(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
 __device__ __forceinline__ float wave_min_f(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off));
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+  v = row_min(v);
+  return fminf(fminf(lane_f(v, 0), lane_f(v, 16)), fminf(lane_f(v, 32), lane_f(v, 48)));
 }
 __device__ __forceinline__ float wave_max_f(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+  v = row_max(v);
+  return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
 }
 
 // Second-order pose statistics of one target lane, from the sums the pair
@@ -714,99 +864,134 @@ __device__ __forceinline__ float wave_sum_f(float v) {
   return v;
 }
 
-template <int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_batchf_pairs(
-    const Rec3F *__restrict__ Z, const Rec3F *__restrict__ S, const BBound *__restrict__ SB, float far_exp,
-    const BItem *__restrict__ items, const int *__restrict__ order, int nitems, unsigned *__restrict__ queue,
+// A block of sources in LDS: what pair_eval<1, 2> reads of a record.
+struct BBlock {
+  float4 a[64], b[64];
+  float c[64];
+};
+__device__ __forceinline__ void block_put(BBlock &s, int lane, const Rec3F &r) {
+  s.a[lane] = make_float4(r.hx, r.hy, r.hz, r.s11);
+  s.b[lane] = make_float4(r.s22, r.s33, r.s12, r.s13);
+  s.c[lane] = r.s23;
+}
+__device__ __forceinline__ void full_pair(const Rec3F &z, const BBlock &s, int j, float *acc) {
+  const float4 a = s.a[j], b = s.b[j];
+  Rec3F q;
+  q.hx = a.x; q.hy = a.y; q.hz = a.z; q.s11 = a.w;
+  q.s22 = b.x; q.s33 = b.y; q.s12 = b.z; q.s13 = b.w;
+  q.s23 = s.c[j];
+  pair_eval<1, 2>(z, q, acc);
+}
+
+// Bound by FP32 issue once the units fill the chip, by the longest unit before:
+// a registration's 90 passes of 64 trials took 353 us each on average with one
+// wave per 64 targets streaming through SGPRs, 74 with the blocks shared.
+template <int S>
+__global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_batchf_pairs(
+    const Rec3I *__restrict__ T, const BCov *__restrict__ TC, const BTrial *__restrict__ trials,
+    const BRef *__restrict__ ref, const Rec3F *__restrict__ Sr, const BBound *__restrict__ SB, float far_exp,
+    const BItem *__restrict__ items, const int *__restrict__ order, int nunits, unsigned *__restrict__ queue,
     const int *__restrict__ done, double *__restrict__ part) {
-  __shared__ int s_p;
-  __shared__ double red[W][kRefStat];
+  constexpr int NA = 10;
+  __shared__ int s_slot[2];
+  __shared__ BBlock s_src[S];
+  __shared__ float s_x[S * NA * 64];
+  __shared__ double s_tot[NA * 64];
+  __shared__ unsigned long long s_near[S];  // a window's blocks that are not far: 64 per wave
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (;;) {
-    if (threadIdx.x == 0) s_p = (int)atomicAdd(queue, 1u);
-    __syncthreads();
-    const int p = __builtin_amdgcn_readfirstlane(s_p);
-    __syncthreads();
-    if (p >= nitems) break;
-    const int idx = __builtin_amdgcn_readfirstlane(order[p]);
-    const BItem it = items[idx];
+  UnitQueue uq(queue, s_slot);
+  for (int p; (p = uq.take(nunits)) < nunits; uq.publish(nunits)) {
+    const int code = __builtin_amdgcn_readfirstlane(order[p]), u = code & 3;
+    const BItem it = items[code >> 2];
     if (done[it.trial]) continue;
-    const int ti = it.t0 + wave * 64 + lane;
-    const bool valid = (wave * 64 + lane) < it.tn;
-    const Rec3F pz = Z[valid ? ti : it.t0];
-    double dacc[10];
+    const bool valid = u * 64 + lane < it.tn;
+    const int ti = valid ? it.t0 + u * 64 + lane : it.t0;
+    const Rec3F pz = batchf_target(T[ti], TC[ti], ref[it.trial], trials[it.trial].c);
+    double d[(NA + S - 1) / S];
 #pragma unroll
-    for (int a = 0; a < 10; ++a) dacc[a] = 0.0;
-    const int s_end = it.s0 + it.sn;
-    const int s_run = wave * 64 < it.tn ? s_end : it.s0;  // idle waves skip the pairs
-    // the wave's targets: bounding box and largest eigenvalue bound (lanes
-    // past the tile hold the tile's first target)
+    for (int i = 0; i * S < NA; ++i) d[i] = 0.0;
+    // the targets' bounding box and largest eigenvalue bound (lanes past the
+    // tile hold the tile's first target)
     const float zlo0 = wave_min_f(pz.hx), zlo1 = wave_min_f(pz.hy), zlo2 = wave_min_f(pz.hz);
     const float zhi0 = wave_max_f(pz.hx), zhi1 = wave_max_f(pz.hy), zhi2 = wave_max_f(pz.hz);
     const float zlam = wave_max_f(pz.pad0);
-    Rec3F qa = S[it.s0], qb = S[min(it.s0 + 1, s_end - 1)];  // it.sn >= 1
-    bool primed = true;  // qa, qb hold records j0 and j0 + 1
-    for (int j0 = it.s0, blk = it.blk; j0 < s_run; j0 += kBSub, ++blk) {
-      const BBound bd = SB[blk];
-      const float g0 = fmaxf(0.0f, fmaxf(bd.lo[0] - zhi0, zlo0 - bd.hi[0]));
-      const float g1 = fmaxf(0.0f, fmaxf(bd.lo[1] - zhi1, zlo1 - bd.hi[1]));
-      const float g2 = fmaxf(0.0f, fmaxf(bd.lo[2] - zhi2, zlo2 - bd.hi[2]));
-      const float gap2 = fmaf(g0, g0, fmaf(g1, g1, g2 * g2));
-      if (__builtin_amdgcn_readfirstlane(gap2 > far_exp * (zlam + bd.lam) ? 1 : 0)) {
-        primed = false;  // far from every target of the wave
-        continue;
+    const int nblk = (it.sn + kBSub - 1) / kBSub;
+    for (int w0 = 0; w0 < nblk; w0 += 64 * S) {
+      if (w0 > 0) __syncthreads();  // the last window's masks have been read
+      const int bt = w0 + (int)threadIdx.x;
+      bool near = false;
+      if (bt < nblk) {
+        const BBound bd = SB[it.blk + bt];
+        const float g0 = fmaxf(0.0f, fmaxf(bd.lo[0] - zhi0, zlo0 - bd.hi[0]));
+        const float g1 = fmaxf(0.0f, fmaxf(bd.lo[1] - zhi1, zlo1 - bd.hi[1]));
+        const float g2 = fmaxf(0.0f, fmaxf(bd.lo[2] - zhi2, zlo2 - bd.hi[2]));
+        const float gap2 = fmaf(g0, g0, fmaf(g1, g1, g2 * g2));
+        near = !(gap2 > far_exp * (zlam + bd.lam));
       }
-      if (!primed) {
-        qa = S[j0];
-        qb = S[min(j0 + 1, s_end - 1)];
-        primed = true;
-      }
-      float acc[10];
+      const unsigned long long nm = __ballot(near);
+      if (lane == 0) s_near[wave] = nm;
+      __syncthreads();
+      int total = 0;
 #pragma unroll
-      for (int a = 0; a < 10; ++a) acc[a] = 0.0f;
-      const int j1 = min(j0 + kBSub, s_end);
-      for (int j = j0; j < j1; ++j) {
-        const Rec3F q = qa;
-        qa = qb;
-        qb = S[min(j + 2, s_end - 1)];
-        pair_eval<1, 2>(pz, q, acc);
-      }
+      for (int k = 0; k < S; ++k) total += __popcll(s_near[k]);
+      total = __builtin_amdgcn_readfirstlane(total);
+      // the wave's blocks: set bits wave, wave + S, ... of the masks in order
+      int mi = -1, skip = wave;
+      unsigned long long m = 0;
+      for (int k0 = 0; k0 < total; k0 += S) {
+        const bool has = k0 + wave < total;
+        float acc[NA];
 #pragma unroll
-      for (int a = 0; a < 10; ++a) dacc[a] += (double)acc[a];
-    }
-    {
-      double r[7] = {0, 0, 0, 0, 0, 0, 0};
-      const double zero[3] = {0.0, 0.0, 0.0};
-      if (valid) pose_contrib(pz, dacc, zero, r);
+        for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
+        if (has) {
+          for (int c; skip >= (c = __popcll(m)); skip -= c) {
+            ++mi;
+            const unsigned long long v = s_near[mi];
+            m = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)v) |
+                (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32)) << 32;
+          }
+          for (; skip > 0; --skip) m &= m - 1;
+          const int b = w0 + 64 * mi + __builtin_ctzll(m);
+          skip = S;
+          const int n = min(kBSub, it.sn - b * kBSub);
+          block_put(s_src[wave], lane, Sr[it.s0 + b * kBSub + min(lane, n - 1)]);
+          wave_lds_fence();
+          int j = 0;
+          for (; j + 4 <= n; j += 4) {
 #pragma unroll
-      for (int a = 0; a < 7; ++a) {
-        const double v = wave_sum(r[a]);
-        if (lane == 0) red[wave][a] = v;
-      }
-    }
-    {
-      const float z[3] = {pz.hx, pz.hy, pz.hz};
-      float af[10];
-#pragma unroll
-      for (int a = 0; a < 10; ++a) af[a] = (float)dacc[a];
-      int q = 7;
-#pragma unroll
-      for (int i = 0; i < 6; ++i)
-#pragma unroll
-        for (int j = i; j < 6; ++j) {
-          const float v = wave_sum_f(valid ? pose_hessian_entry(i, j, z, af) : 0.0f);
-          if (lane == 0) red[wave][q] = (double)v;
-          ++q;
+            for (int k = 0; k < 4; ++k) full_pair(pz, s_src[wave], j + k, acc);
+          }
+          for (; j < n; ++j) full_pair(pz, s_src[wave], j, acc);
+          wave_lds_fence();
         }
+        add_blocks<S, NA>(s_x, acc, has, min(S, total - k0), wave, lane, d);
+      }
     }
-    __syncthreads();
-    if (threadIdx.x < kRefStat) {
-      double v = red[0][threadIdx.x];
+    double dacc[NA];
+    share_sums<S, NA>(d, s_tot, wave, lane, dacc);
+    double r[7] = {0, 0, 0, 0, 0, 0, 0};
+    const double zero[3] = {0.0, 0.0, 0.0};
+    if (valid) pose_contrib(pz, dacc, zero, r);
+    double *o = part + (size_t)(it.u0 + u) * kStat;
 #pragma unroll
-      for (int w = 1; w < W; ++w) v += red[w][threadIdx.x];
-      part[(size_t)idx * kStat + threadIdx.x] = v;
+    for (int a = 0; a < 7; ++a) {
+      if (a % S != wave) continue;  // uniform
+      const double v = wave_sum(r[a]);
+      if (lane == 0) o[a] = v;
     }
-    __syncthreads();
+    const float z[3] = {pz.hx, pz.hy, pz.hz};
+    float af[10];
+#pragma unroll
+    for (int a = 0; a < 10; ++a) af[a] = (float)dacc[a];
+    int q = 7;
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int j = i; j < 6; ++j, ++q) {
+        if (q % S != wave) continue;  // uniform
+        const float v = wave_sum_f(valid ? pose_hessian_entry(i, j, z, af) : 0.0f);
+        if (lane == 0) o[q] = (double)v;
+      }
   }
 }
 
@@ -950,23 +1135,14 @@ __device__ bool newton_inverse(const double *st, const double *cR, const double 
 // in LDS a block of items at a time, thread a summing statistic a in item
 // order, into fold[k]; re-arms the queue.
 __global__ __launch_bounds__(kUpd) void k_batchf_fold(const double *__restrict__ part,
-                                                      const int *__restrict__ titem, int k0, int k1,
+                                                      int W, const int *__restrict__ titem, int k0, int k1,
                                                       const int *__restrict__ done,
                                                       unsigned *__restrict__ queue, double *__restrict__ fold) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0u;
   const int k = k0 + blockIdx.x;
   if (k >= k1 || done[k]) return;
   __shared__ double s_part[kUpdItems * kStat];
-  const int i0 = titem[k], i1 = titem[k + 1];
-  double acc = 0.0;
-  for (int ib = i0; ib < i1; ib += kUpdItems) {
-    const int nb = min(kUpdItems, i1 - ib);
-    for (int e = threadIdx.x; e < nb * kStat; e += kUpd) s_part[e] = part[(size_t)ib * kStat + e];
-    __syncthreads();
-    if (threadIdx.x < kRefStat)
-      for (int i = 0; i < nb; ++i) acc += s_part[i * kStat + threadIdx.x];
-    __syncthreads();
-  }
+  const double acc = fold_items(part, titem[k], titem[k + 1], W, kRefStat, s_part);
   if (threadIdx.x < kRefStat) fold[(size_t)k * kStat + threadIdx.x] = acc;
 }
 
@@ -1086,28 +1262,26 @@ __global__ __launch_bounds__(256) void k_batchf_update(const double *__restrict_
 constexpr int kLevels = 3;
 constexpr int kLevelStep[kLevels] = {1, 4, 2};
 struct BLevel {
-  int ntgt = 0, nsrc = 0, nitems = 0;
+  int ntgt = 0, nsrc = 0, nitems = 0, nunits = 0;
   Rec3I *dT = nullptr;       // targets (all trials), relative to each trial's centroid
-  BZ *dZ = nullptr;          // per-iteration targets in each trial's source frame
-  int *dtgt_trial = nullptr; // trial of each target
   BSrc *dS = nullptr;        // sources (all trials), as given
   BItem *ditems = nullptr;
-  int *dorder = nullptr;     // queue position -> item, longest first
-  int *dident = nullptr;     // identity order for one-trial launches
-  int *dactive = nullptr;    // the running trials' items only, longest first (tail passes)
+  int *dorder = nullptr;     // queue: the items' units (4 item + piece), longest item first
+  int *dident = nullptr;     // units in item order, for one-trial launches
+  int *dactive = nullptr;    // the running trials' units only, longest first (tail passes)
   int *dtitem = nullptr;     // CSR: items of trial k are [titem[k], titem[k+1])
   int *dttgt = nullptr;      // CSR: targets of trial k are [ttgt[k], ttgt[k+1])
   unsigned *dnn = nullptr;   // per target: smallest |d|^2 of the current pass (float bits)
-  double *dpart = nullptr;   // per-item statistics
-  size_t items_cap = 0;      // capacity of ditems / dorder / dident / dpart
+  double *dpart = nullptr;   // per-unit statistics
+  size_t items_cap = 0, units_cap = 0;  // capacity of ditems; of dorder / dident / dactive / dpart
   std::vector<int> tb, nt, sb, ns;  // per trial: target / source base and count
   std::vector<int> bb;              // per trial: first 64-source block (prefix of ceil(ns / 64))
   int nblocks = 0;                  // 64-source blocks of the level
-  std::vector<int> titem;
-  std::vector<int> horder, hitem_trial;  // host copies: queue order; trial of each item
+  std::vector<int> titem, tunit;  // CSR per trial: items, units
+  std::vector<int> horder, hitem_trial;  // host copies: queue; trial of each item
   long long pairs = 0;              // target x source pairs of one full iteration
   // launch shape of this level's persistent pair kernels
-  int waves = 4;                        // waves per workgroup: target tile = 64 * waves
+  int waves = 4;                        // units per target tile: tile = 64 * waves targets
   int chunks[kClasses] = {1, 1, 2, 4};  // source chunks per target tile, per size class
   int grid_waves = 8192;                // resident waves
 };
@@ -1131,7 +1305,6 @@ struct dugma_batch {
   // covariances times the level's point step)
   BCov *dTC[kLevels] = {};                  // per target: covariance
   Rec3F *dSF[kLevels] = {};                 // per source: position and covariance (static)
-  Rec3F *dZF[kLevels] = {};                 // per target at each pass: in the trial's source frame
   BBound *dSB[kLevels] = {};                // per 64-source block: box and eigenvalue bound
   float far_exp = kFarExp;                  // skip threshold (infinite: no skip)
   BRef *dref = nullptr;                     // per trial: optimiser state
@@ -1143,7 +1316,7 @@ struct dugma_batch {
 };
 
 static void free_level(BLevel &L) {
-  void *ptrs[] = {L.dT, L.dZ, L.dtgt_trial, L.dS, L.ditems, L.dorder, L.dident, L.dactive,
+  void *ptrs[] = {L.dT, L.dS, L.ditems, L.dorder, L.dident, L.dactive,
                   L.dtitem, L.dttgt, L.dnn, L.dpart};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -1153,7 +1326,7 @@ static void free_batch(dugma_batch *b) {
   if (!b) return;
   for (int l = 0; l < kLevels; ++l) {
     free_level(b->lv[l]);
-    void *lp[] = {b->dTC[l], b->dSF[l], b->dZF[l], b->dSB[l]};
+    void *lp[] = {b->dTC[l], b->dSF[l], b->dSB[l]};
     for (void *p : lp)
       if (p) (void)hipFree(p);
   }
@@ -1183,10 +1356,13 @@ static int make_items(dugma_batch *b, BLevel &L) {
   const int K = b->ntrials, tile_t = 64 * L.waves;
   std::vector<BItem> items;
   L.titem.assign(K + 1, 0);
+  L.tunit.assign(K + 1, 0);
+  int nu = 0;
   L.bb.assign(K, 0);
   L.nblocks = 0;
   for (int k = 0; k < K; ++k) {
     L.titem[k] = (int)items.size();
+    L.tunit[k] = nu;
     L.bb[k] = L.nblocks;
     const int nt = L.nt[k], ns = L.ns[k];
     L.nblocks += (ns + kBSub - 1) / kBSub;
@@ -1204,40 +1380,68 @@ static int make_items(dugma_batch *b, BLevel &L) {
         it.s0 = L.sb[k] + s0;
         it.sn = std::min(tile_s, ns - s0);
         it.blk = L.bb[k] + s0 / kBSub;
+        it.u0 = (int)items.size() * L.waves;
+        it.nu = (it.tn + 63) / 64;
+        nu += it.nu;
         items.push_back(it);
       }
   }
   L.titem[K] = (int)items.size();
-  std::vector<int> order(items.size()), ident(items.size());
+  L.tunit[K] = nu;
+  std::vector<int> order(items.size());
   std::iota(order.begin(), order.end(), 0);
-  std::iota(ident.begin(), ident.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int u, int v) {
     return (long long)items[u].tn * items[u].sn > (long long)items[v].tn * items[v].sn;
   });
+  std::vector<int> queue, ident;
+  queue.reserve(nu);
+  ident.reserve(nu);
+  // whole 4-unit tiles stay on multiples of 4 (k_batch_pairs_wide's
+  // workgroups): the units of partial ones wait until there are 4
+  std::vector<int> rest;
+  for (int i : order) {
+    std::vector<int> &to = items[i].nu == kWideUnits ? queue : rest;
+    for (int u = 0; u < items[i].nu; ++u) to.push_back(4 * i + u);
+    if (&to == &rest && rest.size() >= kWideUnits) {
+      queue.insert(queue.end(), rest.begin(), rest.begin() + kWideUnits);
+      rest.erase(rest.begin(), rest.begin() + kWideUnits);
+    }
+  }
+  queue.insert(queue.end(), rest.begin(), rest.end());
+  for (int i = 0; i < (int)items.size(); ++i)
+    for (int u = 0; u < items[i].nu; ++u) ident.push_back(4 * i + u);
+  int rc;
   if (items.size() > L.items_cap) {
-    void *old[] = {L.ditems, L.dorder, L.dident, L.dactive, L.dpart};
-    for (void *p : old)
-      if (p) (void)hipFree(p);
+    if (L.ditems) (void)hipFree(L.ditems);
     L.ditems = nullptr;
-    L.dorder = L.dident = L.dactive = nullptr;
-    L.dpart = nullptr;
     L.items_cap = 0;
-    int rc;
-    if ((rc = bmalloc(&L.ditems, items.size())) || (rc = bmalloc(&L.dorder, items.size())) ||
-        (rc = bmalloc(&L.dident, items.size())) || (rc = bmalloc(&L.dactive, items.size())) ||
-        (rc = bmalloc(&L.dpart, items.size() * kStat)))
-      return rc;
+    if ((rc = bmalloc(&L.ditems, items.size()))) return rc;
     L.items_cap = items.size();
   }
+  const size_t nrec = items.size() * L.waves;
+  if (nrec > L.units_cap) {
+    void *old[] = {L.dorder, L.dident, L.dactive, L.dpart};
+    for (void *p : old)
+      if (p) (void)hipFree(p);
+    L.dorder = L.dident = L.dactive = nullptr;
+    L.dpart = nullptr;
+    L.units_cap = 0;
+    if ((rc = bmalloc(&L.dorder, nrec)) || (rc = bmalloc(&L.dident, nrec)) || (rc = bmalloc(&L.dactive, nrec)) ||
+        (rc = bmalloc(&L.dpart, nrec * kStat)))
+      return rc;
+    L.units_cap = nrec;
+  }
+  if (nrec > 0) DUGMA_HIP(hipMemset(L.dpart, 0, nrec * kStat * sizeof(double)));
   L.hitem_trial.resize(items.size());
   for (size_t i = 0; i < items.size(); ++i) L.hitem_trial[i] = items[i].trial;
-  L.horder = order;
   L.nitems = (int)items.size();
+  L.nunits = nu;
   if (!items.empty()) {
     DUGMA_HIP(hipMemcpy(L.ditems, items.data(), items.size() * sizeof(BItem), hipMemcpyHostToDevice));
-    DUGMA_HIP(hipMemcpy(L.dorder, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice));
+    DUGMA_HIP(hipMemcpy(L.dorder, queue.data(), queue.size() * sizeof(int), hipMemcpyHostToDevice));
     DUGMA_HIP(hipMemcpy(L.dident, ident.data(), ident.size() * sizeof(int), hipMemcpyHostToDevice));
   }
+  L.horder = std::move(queue);
   DUGMA_HIP(hipMemcpy(L.dtitem, L.titem.data(), L.titem.size() * sizeof(int), hipMemcpyHostToDevice));
   return DUGMA_OK;
 }
@@ -1252,7 +1456,7 @@ static int make_all_items(dugma_batch *b) {
 struct LevelHost {
   std::vector<Rec3I> tg;
   std::vector<BSrc> sr;
-  std::vector<int> ttrial, ttgt;
+  std::vector<int> ttgt;
 };
 
 static int upload_level(dugma_batch *b, BLevel &L, const LevelHost &H) {
@@ -1260,8 +1464,7 @@ static int upload_level(dugma_batch *b, BLevel &L, const LevelHost &H) {
   L.ntgt = (int)H.tg.size();
   L.nsrc = (int)H.sr.size();
   int rc;
-  if ((rc = bmalloc(&L.dT, H.tg.size())) || (rc = bmalloc(&L.dZ, H.tg.size())) ||
-      (rc = bmalloc(&L.dtgt_trial, H.ttrial.size())) || (rc = bmalloc(&L.dS, H.sr.size())) ||
+  if ((rc = bmalloc(&L.dT, H.tg.size())) || (rc = bmalloc(&L.dS, H.sr.size())) ||
       (rc = bmalloc(&L.dtitem, (size_t)K + 1)) || (rc = bmalloc(&L.dttgt, (size_t)K + 1)) ||
       (rc = bmalloc(&L.dnn, H.tg.size())))
     return rc;
@@ -1270,7 +1473,6 @@ static int upload_level(dugma_batch *b, BLevel &L, const LevelHost &H) {
     const void *h;
     size_t n;
   } ups[] = {{L.dT, H.tg.data(), H.tg.size() * sizeof(Rec3I)},
-             {L.dtgt_trial, H.ttrial.data(), H.ttrial.size() * sizeof(int)},
              {L.dS, H.sr.data(), H.sr.size() * sizeof(BSrc)},
              {L.dttgt, H.ttgt.data(), H.ttgt.size() * sizeof(int)}};
   for (const Up &u : ups)
@@ -1446,7 +1648,6 @@ static int build_batch(int ntrials, const int *N, const int *M, const double *co
           vt += tv[i];
         }
         h.tg.push_back(r);
-        h.ttrial.push_back(k);
       }
       L.nt[k] = (int)h.tg.size() - L.tb[k];
       L.sb[k] = (int)h.sr.size();
@@ -1537,18 +1738,65 @@ extern "C" int dugma_batch_info(const dugma_batch *b, int *ntrials, int *nitems,
   return DUGMA_OK;
 }
 
-template <int W>
+// Waves that share a unit's source blocks (no result depends on it): the fewer
+// units, the more.  kWaveSlots: 256 CUs x 4 SIMDs x 8.  Whole runs on one
+// MI355X: isotropic coarse iterations (121 passes), 20 trials (230 units)
+// 7.9 / 6.3 / 6.0 ms with 4 / 8 / 16 waves, 256 (2,900) 14.0 / 13.3 / 15.0, 1,024
+// (11,700) 33.9 / 35.3; 12 full-cloud iterations of 256 trials (24,000 units)
+// 10.6 / 10.7 and 11.2 with a wave per unit, of 1,024 (95,000) 39 / 40 and 35;
+// the whole schedule with refinement, 1,024 trials, 78 / 80.
+constexpr int kWaveSlots = 8192;
+static int iso_waves(const BLevel &L) {
+  return L.nunits < kWaveSlots / 16 ? 16 : L.nunits < kWaveSlots ? 8 : L.nunits < 5 * kWaveSlots ? 4 : 1;
+}
+static int refine_waves(const BLevel &L) { return L.nunits < 4 * kWaveSlots ? 8 : 4; }
+
+// Workgroups of a pair kernel: one per unit (the dispatcher hands them out
+// faster than the queue's counter: 2,048 trials, 4 waves a unit, the whole
+// registration in 138 ms against 160 with 2,048 persistent workgroups), at most
+// kDispatch times the shape's resident waves or what the caller asks for; they
+// then take the rest from the queue.
+constexpr int kDispatch = 64;
+static int unit_grid(const BLevel &L, int grid, int s, int ni) {
+  if (grid <= 0) grid = (int)std::min<long long>(ni, std::max(1LL, (long long)kDispatch * L.grid_waves / s));
+  return std::min(grid, ni);
+}
+
+template <int S>
+static void launch_pairs_s(dugma_batch *b, const BLevel &L, int grid, const int *order, int ni, bool sigma,
+                           bool energy) {
+  const dim3 g(unit_grid(L, grid, S, ni)), blk(64 * S);
+  if (energy)  // the energy pass after the iterations (no sigma measurement)
+    hipLaunchKernelGGL((k_batch_pairs<S, false, true>), g, blk, 0, b->stream, L.dT, b->dtrials, L.dS, L.ditems,
+                       order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
+  else if (sigma)
+    hipLaunchKernelGGL((k_batch_pairs<S, true, false>), g, blk, 0, b->stream, L.dT, b->dtrials, L.dS, L.ditems,
+                       order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
+  else
+    hipLaunchKernelGGL((k_batch_pairs<S, false, false>), g, blk, 0, b->stream, L.dT, b->dtrials, L.dS, L.ditems,
+                       order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
+}
+static void launch_pairs_wide(dugma_batch *b, const BLevel &L, int grid, const int *order, int ni, bool sigma,
+                              bool energy) {
+  const dim3 g(unit_grid(L, grid, kWideUnits, (ni + kWideUnits - 1) / kWideUnits)), blk(64 * kWideUnits);
+  if (energy)
+    hipLaunchKernelGGL((k_batch_pairs_wide<false, true>), g, blk, 0, b->stream, L.dT, b->dtrials, L.dS, L.ditems,
+                       order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
+  else if (sigma)
+    hipLaunchKernelGGL((k_batch_pairs_wide<true, false>), g, blk, 0, b->stream, L.dT, b->dtrials, L.dS, L.ditems,
+                       order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
+  else
+    hipLaunchKernelGGL((k_batch_pairs_wide<false, false>), g, blk, 0, b->stream, L.dT, b->dtrials, L.dS, L.ditems,
+                       order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
+}
 static void launch_pairs(dugma_batch *b, const BLevel &L, int grid, const int *order, int ni, bool sigma,
                          bool energy = false) {
-  if (energy)  // the energy pass after the iterations (no sigma measurement)
-    hipLaunchKernelGGL((k_batch_pairs<W, false, true>), dim3(grid), dim3(64 * W), 0, b->stream, L.dT, L.dZ,
-                       L.dS, L.ditems, order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
-  else if (sigma)
-    hipLaunchKernelGGL((k_batch_pairs<W, true, false>), dim3(grid), dim3(64 * W), 0, b->stream, L.dT, L.dZ,
-                       L.dS, L.ditems, order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
-  else
-    hipLaunchKernelGGL((k_batch_pairs<W, false, false>), dim3(grid), dim3(64 * W), 0, b->stream, L.dT, L.dZ,
-                       L.dS, L.ditems, order, ni, b->dqueue, b->ddone, L.dnn, L.dpart);
+  switch (iso_waves(L)) {
+    case 1: launch_pairs_wide(b, L, grid, order, ni, sigma, energy); break;
+    case 4: launch_pairs_s<4>(b, L, grid, order, ni, sigma, energy); break;
+    case 8: launch_pairs_s<8>(b, L, grid, order, ni, sigma, energy); break;
+    default: launch_pairs_s<16>(b, L, grid, order, ni, sigma, energy); break;
+  }
 }
 
 // One iteration of trials [k0, k1) on level l.  grid: workgroups of the
@@ -1556,31 +1804,16 @@ static void launch_pairs(dugma_batch *b, const BLevel &L, int grid, const int *o
 static int launch_iteration(dugma_batch *b, int l, int k0, int k1, const BParams &bp,
                             bool one_trial, int grid, const int *order_in = nullptr, int ni_in = 0) {
   const BLevel &L = b->lv[l];
-  int t0 = 0, t1 = L.ntgt;
   const int *order = order_in ? order_in : L.dorder;
-  int ni = order_in ? ni_in : L.nitems;
+  int ni = order_in ? ni_in : L.nunits;
   if (one_trial) {
-    // items of trial k0 are contiguous: [titem[k0], titem[k0+1])
-    const int i0 = L.titem[k0];
-    ni = L.titem[k0 + 1] - i0;
-    order = L.dident + i0;
-    t0 = L.tb[k0];
-    t1 = t0 + L.nt[k0];
+    // units of trial k0 are contiguous: [tunit[k0], tunit[k0+1])
+    order = L.dident + L.tunit[k0];
+    ni = L.tunit[k0 + 1] - L.tunit[k0];
   }
-  if (t1 > t0)
-    hipLaunchKernelGGL(k_batch_transform, dim3((t1 - t0 + 255) / 256), dim3(256), 0, b->stream, L.dT,
-                       L.dtgt_trial, t0, t1, b->dtrials, b->ddone, L.dZ);
-  if (ni > 0) {
-    if (grid <= 0) grid = std::max(1, L.grid_waves / L.waves);
-    grid = std::min(grid, ni);
-    switch (L.waves) {
-      case 1: launch_pairs<1>(b, L, grid, order, ni, bp.sigma != 0); break;
-      case 2: launch_pairs<2>(b, L, grid, order, ni, bp.sigma != 0); break;
-      default: launch_pairs<4>(b, L, grid, order, ni, bp.sigma != 0); break;
-    }
-  }
-  hipLaunchKernelGGL(k_batch_fold, dim3(k1 - k0), dim3(kUpd), 0, b->stream, L.dpart, L.dtitem, L.dttgt, k0, k1,
-                     b->dtrials, b->ddone, b->dqueue, L.dnn, b->dfold, bp.sigma);
+  if (ni > 0) launch_pairs(b, L, grid, order, ni, bp.sigma != 0);
+  hipLaunchKernelGGL(k_batch_fold, dim3(k1 - k0), dim3(kUpd), 0, b->stream, L.dpart, L.waves, L.dtitem, L.dttgt,
+                     k0, k1, b->dtrials, b->ddone, b->dqueue, L.dnn, b->dfold, bp.sigma);
   hipLaunchKernelGGL(k_batch_update, dim3((k1 - k0 + 63) / 64), dim3(64), 0, b->stream, b->dfold, k0, k1,
                      b->dtrials, b->ddone, bp);
   DUGMA_HIP(hipGetLastError());
@@ -1589,15 +1822,15 @@ static int launch_iteration(dugma_batch *b, int l, int k0, int k1, const BParams
 
 // The tail of a run: once at most a sixteenth of the trials are still
 // running, passes are launched directly (not from the captured graph) over
-// a queue that holds only those trials' items, in the same longest-first
+// a queue that holds only those trials' units, in the same longest-first
 // order, rebuilt whenever the running count has halved again.  A pass then
-// no longer takes every finished trial's items off the queue (on the fine
+// no longer takes every finished trial's units off the queue (on the fine
 // level, 4,096 trials, a pass with every trial finished still took 1.2 ms).
-// Results do not change: an item writes only its own statistics slot, and
-// a finished trial's items are skipped either way.
+// Results do not change: a unit writes only its own statistics record, and
+// a finished trial's units are skipped either way.
 struct TailQueue {
   int last_active = -1;  // running trials when the queue was last rebuilt
-  int n = 0;             // items in the level's dactive (0: the full queue)
+  int n = 0;             // units in the level's dactive (0: the full queue)
   // hd: the done flags just read back
   int update(dugma_batch *b, const BLevel &L, const std::vector<int> &hd) {
     const int K = b->ntrials;
@@ -1608,7 +1841,7 @@ struct TailQueue {
     std::vector<int> q;
     q.reserve(L.horder.size());
     for (int p : L.horder)
-      if (!hd[L.hitem_trial[p]]) q.push_back(p);
+      if (!hd[L.hitem_trial[p >> 2]]) q.push_back(p);
     last_active = active;
     n = (int)q.size();
     if (n > 0) {
@@ -1626,19 +1859,9 @@ static int energy_pass(dugma_batch *b) {
   const BLevel &L = b->lv[0];
   const int K = b->ntrials;
   hipLaunchKernelGGL(k_batch_fill, dim3((K + 255) / 256), dim3(256), 0, b->stream, (unsigned *)b->ddone, K, 0u);
-  if (L.ntgt > 0)
-    hipLaunchKernelGGL(k_batch_transform, dim3((L.ntgt + 255) / 256), dim3(256), 0, b->stream, L.dT,
-                       L.dtgt_trial, 0, L.ntgt, b->dtrials, b->ddone, L.dZ);
-  if (L.nitems > 0) {
-    const int grid = std::min(std::max(1, L.grid_waves / L.waves), L.nitems);
-    switch (L.waves) {
-      case 1: launch_pairs<1>(b, L, grid, L.dorder, L.nitems, false, true); break;
-      case 2: launch_pairs<2>(b, L, grid, L.dorder, L.nitems, false, true); break;
-      default: launch_pairs<4>(b, L, grid, L.dorder, L.nitems, false, true); break;
-    }
-  }
-  hipLaunchKernelGGL(k_batch_energy, dim3((K + 255) / 256), dim3(256), 0, b->stream, L.dpart, L.dtitem, K,
-                     b->dtrials, b->dqueue);
+  if (L.nunits > 0) launch_pairs(b, L, 0, L.dorder, L.nunits, false, true);
+  hipLaunchKernelGGL(k_batch_energy, dim3((K + 255) / 256), dim3(256), 0, b->stream, L.dpart, L.waves,
+                     L.dtitem, K, b->dtrials, b->dqueue);
   DUGMA_HIP(hipGetLastError());
   return DUGMA_OK;
 }
@@ -1673,42 +1896,33 @@ static int start_trials(dugma_batch *b, const double *R0, const double *t0, bool
   return DUGMA_OK;
 }
 
-template <int W>
-static void launch_pairsf(dugma_batch *b, int l, int grid, const int *order, int ni) {
+template <int S>
+static void launch_pairsf_s(dugma_batch *b, int l, int grid, const int *order, int ni) {
   const BLevel &L = b->lv[l];
-  hipLaunchKernelGGL((k_batchf_pairs<W>), dim3(grid), dim3(64 * W), 0, b->stream, b->dZF[l], b->dSF[l],
-                     b->dSB[l], b->far_exp, L.ditems, order, ni, b->dqueue, b->ddone, L.dpart);
+  hipLaunchKernelGGL((k_batchf_pairs<S>), dim3(unit_grid(L, grid, S, ni)), dim3(64 * S), 0, b->stream, L.dT,
+                     b->dTC[l], b->dtrials, b->dref, b->dSF[l], b->dSB[l], b->far_exp, L.ditems, order, ni,
+                     b->dqueue, b->ddone, L.dpart);
 }
 
-// One refinement pass of trials [k0, k1) on level l: transform at the
-// candidate poses, pairs, optimiser step.
+// One refinement pass of trials [k0, k1) on level l: pairs at the candidate
+// poses, optimiser step.
 static int launch_refine(dugma_batch *b, int l, int k0, int k1, const RParams &rp, bool one_trial, int grid,
                          const int *order_in = nullptr, int ni_in = 0) {
   const BLevel &L = b->lv[l];
-  int t0 = 0, t1 = L.ntgt;
   const int *order = order_in ? order_in : L.dorder;
-  int ni = order_in ? ni_in : L.nitems;
+  int ni = order_in ? ni_in : L.nunits;
   if (one_trial) {
-    const int i0 = L.titem[k0];
-    ni = L.titem[k0 + 1] - i0;
-    order = L.dident + i0;
-    t0 = L.tb[k0];
-    t1 = t0 + L.nt[k0];
+    order = L.dident + L.tunit[k0];
+    ni = L.tunit[k0 + 1] - L.tunit[k0];
   }
-  if (t1 > t0)
-    hipLaunchKernelGGL(k_batchf_transform, dim3((t1 - t0 + 255) / 256), dim3(256), 0, b->stream, L.dT, b->dTC[l],
-                       L.dtgt_trial, t0, t1, b->dtrials, b->dref, b->ddone, b->dZF[l]);
   if (ni > 0) {
-    if (grid <= 0) grid = std::max(1, L.grid_waves / L.waves);
-    grid = std::min(grid, ni);
-    switch (L.waves) {
-      case 1: launch_pairsf<1>(b, l, grid, order, ni); break;
-      case 2: launch_pairsf<2>(b, l, grid, order, ni); break;
-      default: launch_pairsf<4>(b, l, grid, order, ni); break;
-    }
+    if (refine_waves(L) == 4)
+      launch_pairsf_s<4>(b, l, grid, order, ni);
+    else
+      launch_pairsf_s<8>(b, l, grid, order, ni);
   }
-  hipLaunchKernelGGL(k_batchf_fold, dim3(k1 - k0), dim3(kUpd), 0, b->stream, L.dpart, L.dtitem, k0, k1, b->ddone,
-                     b->dqueue, b->dfold);
+  hipLaunchKernelGGL(k_batchf_fold, dim3(k1 - k0), dim3(kUpd), 0, b->stream, L.dpart, L.waves, L.dtitem, k0, k1,
+                     b->ddone, b->dqueue, b->dfold);
   hipLaunchKernelGGL(k_batchf_update, dim3((k1 - k0 + 255) / 256), dim3(256), 0, b->stream, b->dfold, k0, k1,
                      b->dref, b->ddone, rp);
   DUGMA_HIP(hipGetLastError());
@@ -2168,7 +2382,6 @@ extern "C" int dugma_batch_set_covariances(dugma_batch *b, const double *const *
     for (int l = 0; l < kLevels && !rc; ++l) {
       if (!b->dTC[l] && (rc = bmalloc(&b->dTC[l], tcl[l].size()))) break;
       if (!b->dSF[l] && (rc = bmalloc(&b->dSF[l], sfl[l].size()))) break;
-      if (!b->dZF[l] && (rc = bmalloc(&b->dZF[l], tcl[l].size()))) break;
       if (!b->dSB[l] && (rc = bmalloc(&b->dSB[l], sbl[l].size()))) break;
     }
     if (rc) return rc;
