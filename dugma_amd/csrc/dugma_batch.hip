@@ -254,12 +254,6 @@ struct UnitQueue {
   }
 };
 
-// Orders a wave's own LDS writes and reads (no other wave uses them).
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // One round of a unit: each wave's FP32 block sums (where it had a block: nb
 // waves) through LDS to their owners, who add them in block order.
 template <int S, int NA>
@@ -864,25 +858,6 @@ __device__ __forceinline__ float wave_sum_f(float v) {
   return v;
 }
 
-// A block of sources in LDS: what pair_eval<1, 2> reads of a record.
-struct BBlock {
-  float4 a[64], b[64];
-  float c[64];
-};
-__device__ __forceinline__ void block_put(BBlock &s, int lane, const Rec3F &r) {
-  s.a[lane] = make_float4(r.hx, r.hy, r.hz, r.s11);
-  s.b[lane] = make_float4(r.s22, r.s33, r.s12, r.s13);
-  s.c[lane] = r.s23;
-}
-__device__ __forceinline__ void full_pair(const Rec3F &z, const BBlock &s, int j, float *acc) {
-  const float4 a = s.a[j], b = s.b[j];
-  Rec3F q;
-  q.hx = a.x; q.hy = a.y; q.hz = a.z; q.s11 = a.w;
-  q.s22 = b.x; q.s33 = b.y; q.s12 = b.z; q.s13 = b.w;
-  q.s23 = s.c[j];
-  pair_eval<1, 2>(z, q, acc);
-}
-
 // Bound by FP32 issue once the units fill the chip, by the longest unit before:
 // a registration's 90 passes of 64 trials took 353 us each on average with one
 // wave per 64 targets streaming through SGPRs, 74 with the blocks shared.
@@ -894,7 +869,7 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(6, 8))) 
     const int *__restrict__ done, double *__restrict__ part) {
   constexpr int NA = 10;
   __shared__ int s_slot[2];
-  __shared__ BBlock s_src[S];
+  __shared__ LdsRecs<Rec3F, 2> s_src[S];
   __shared__ float s_x[S * NA * 64];
   __shared__ double s_tot[NA * 64];
   __shared__ unsigned long long s_near[S];  // a window's blocks that are not far: 64 per wave
@@ -954,14 +929,14 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(6, 8))) 
           const int b = w0 + 64 * mi + __builtin_ctzll(m);
           skip = S;
           const int n = min(kBSub, it.sn - b * kBSub);
-          block_put(s_src[wave], lane, Sr[it.s0 + b * kBSub + min(lane, n - 1)]);
+          s_src[wave].put(lane, Sr[it.s0 + b * kBSub + min(lane, n - 1)]);
           wave_lds_fence();
           int j = 0;
           for (; j + 4 <= n; j += 4) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) full_pair(pz, s_src[wave], j + k, acc);
+            for (int k = 0; k < 4; ++k) pair_eval<1, 2>(pz, s_src[wave].get(j + k), acc);
           }
-          for (; j < n; ++j) full_pair(pz, s_src[wave], j, acc);
+          for (; j < n; ++j) pair_eval<1, 2>(pz, s_src[wave].get(j), acc);
           wave_lds_fence();
         }
         add_blocks<S, NA>(s_x, acc, has, min(S, total - k0), wave, lane, d);

@@ -179,23 +179,23 @@ __global__ __launch_bounds__(kBlock) void k_transform_src(
 //    bit in LDS for each point that any of the 64 lanes may have a term other
 //    than 0 with.  Bits stand in the streamed points' own order, group by
 //    group.
-// 3. Each wave turns its groups' set bits into a list (LDS), takes 16 entries
-//    at a time -- lane l loads the record of entry l % 16, so every row of 16
-//    lanes holds the 16 records -- and adds their pairs one after another, the
-//    record's words broadcast within the rows by the consuming instruction
-//    (DPP row_newbcast, which issues at the rate of an SGPR operand).  Points
-//    without a bit add exactly 0 for every lane, so the FP32 sums of a group are
-//    those of all its points, in their order.
+// 3. Each wave turns its groups' set bits into a list (LDS), takes 64 entries
+//    at a time -- lane l puts the record of entry l into LDS, every lane then
+//    reads them one by one (LdsRecs) -- and adds their pairs one after another.
+//    Points without a bit add exactly 0 for every lane, so the FP32 sums of a
+//    group are those of all its points, in their order.
 //
-// What bounds it: at 200K x 200K (isotropic, 8-NN sigma) a workgroup lists 3,200
-// of 200,000 streamed points, 1,450 of which any one lane needs; FP32 issue of
-// those pairs and the FP64 flush of their 2,000 sub-tiles.  0.79 ms against
-// 18.4 ms with every pair evaluated (outputs equal to 2e-16).  6,000 x 6,000
-// full covariances: 24 us against 66 (160 listed of 6,000; a chain of
-// dependent loads).  Scalar loads of the listed records (each wave at its own
+// What bounds it: at 200K x 200K (isotropic, 8-NN sigma) a workgroup lists 3,250
+// of 200,000 streamed points, 1,450 of which any one lane needs, in 2,000
+// sub-tiles: VALU issue (407 M wave instructions at 4 cycles: 203 M of the
+// pairs, 80 M of the FP64 flushes, 124 M of finding the points).  0.63 ms;
+// 18.4 ms with every pair evaluated (outputs equal to 2e-16), 0.69 with the
+// records broadcast by DPP row_newbcast (4.5 cycles an operand against 2.5).
+// 6,000 x 6,000 full covariances: 22 us against 66 (160 listed of 6,000; a chain
+// of dependent loads).  Scalar loads of the listed records (each wave at its own
 // addresses) were bound by the scalar cache's misses, 145 cycles per record
 // and CU: 1.86 ms at 200K.
-constexpr int kCap = 256;  // list entries per wave (whole groups at a time)
+constexpr int kCap = 128;  // list entries per wave (whole groups at a time)
 constexpr int kNearBlock = 512;
 constexpr int kNearWaves = kNearBlock / 64;
 constexpr int kRows = 4, kQuads = 16;  // boxes of 16 and of 4 stationary points
@@ -239,37 +239,6 @@ struct NearArg {
   int win;                   // groups per window
 };
 
-// Lane k of the own row of 16, as an operand (k a constant).
-template <int K>
-__device__ __forceinline__ float row_bcast(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xF, 0xF, true));
-}
-template <int K>
-__device__ __forceinline__ void row_bcast(const Rec3F &q, Rec3F &r) {
-  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy); r.hz = row_bcast<K>(q.hz);
-  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly); r.lz = row_bcast<K>(q.lz);
-  r.s11 = row_bcast<K>(q.s11); r.s22 = row_bcast<K>(q.s22); r.s33 = row_bcast<K>(q.s33);
-  r.s12 = row_bcast<K>(q.s12); r.s13 = row_bcast<K>(q.s13); r.s23 = row_bcast<K>(q.s23);
-}
-template <int K>
-__device__ __forceinline__ void row_bcast(const Rec3I &q, Rec3I &r) {
-  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy); r.hz = row_bcast<K>(q.hz);
-  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly); r.lz = row_bcast<K>(q.lz);
-  r.s = row_bcast<K>(q.s);
-}
-template <int K>
-__device__ __forceinline__ void row_bcast(const Rec2F &q, Rec2F &r) {
-  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy);
-  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly);
-  r.s11 = row_bcast<K>(q.s11); r.s12 = row_bcast<K>(q.s12); r.s22 = row_bcast<K>(q.s22);
-}
-template <int K>
-__device__ __forceinline__ void row_bcast(const Rec2I &q, Rec2I &r) {
-  r.hx = row_bcast<K>(q.hx); r.hy = row_bcast<K>(q.hy);
-  r.lx = row_bcast<K>(q.lx); r.ly = row_bcast<K>(q.ly);
-  r.s = row_bcast<K>(q.s);
-}
-
 // The FP32 sums of a group go to the FP64 ones.
 template <int NA>
 __device__ __forceinline__ void flush_group(float *acc, double *dacc) {
@@ -280,39 +249,30 @@ __device__ __forceinline__ void flush_group(float *acc, double *dacc) {
   }
 }
 
-// Pairs of entries K..15 (below n) of the 16 records that each row holds;
-// bit k of first: entry k opens a group.
-template <class Rec, int MODE, int COMP, int NA, int K>
-__device__ __forceinline__ void eval_rows(const Rec &p, const Rec &q, unsigned first, int n, float *acc,
-                                          double *dacc) {
-  if constexpr (K < 16) {
-    if (K >= n) return;  // uniform
-    if ((first >> K) & 1u) flush_group<NA>(acc, dacc);
-    Rec r;
-    row_bcast<K>(q, r);
-    pair_eval<MODE, COMP>(p, r, acc);
-    eval_rows<Rec, MODE, COMP, NA, K + 1>(p, q, first, n, acc, dacc);
-  }
+// Inclusive prefix sum over the 64 lanes (DPP: within rows of 16, then row 0's
+// and 2's totals to the next row, then rows 0 and 1's to rows 2 and 3).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
 }
-
-// Inclusive prefix sum over the 64 lanes.
-__device__ __forceinline__ int wave_scan(int v, int lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_up(v, d, 64);
-    if (lane >= d) v += u;
-  }
-  return v;
+__device__ __forceinline__ int wave_scan(int v) {
+  v = dpp_add<0x111, 0xF>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xF>(v);  // row_shr:2
+  v = dpp_add<0x114, 0xF>(v);  // row_shr:4
+  v = dpp_add<0x118, 0xF>(v);  // row_shr:8
+  v = dpp_add<0x142, 0xA>(v);  // row_bcast:15
+  return dpp_add<0x143, 0xC>(v);  // row_bcast:31
 }
 
 // The pairs of the set bits of the lanes' groups (lane's group: 64 bits, first
 // streamed point js), group by group in lane order: listed in rounds of whole
 // groups, at most kCap entries (a group has at most 64).
 template <class Rec, int MODE, int COMP, int NA>
-__device__ __forceinline__ void walk_groups(const Rec &p, const Rec *__restrict__ Q, unsigned *list, int lane,
-                                            unsigned mlo, unsigned mhi, int js, double *dacc) {
+__device__ __forceinline__ void walk_groups(const Rec &p, const Rec *__restrict__ Q, unsigned *list,
+                                            LdsRecs<Rec, COMP> &recs, int lane, unsigned mlo, unsigned mhi, int js,
+                                            double *dacc) {
   const int cnt = __popc(mlo) + __popc(mhi);
-  const int incl = wave_scan(cnt, lane), excl = incl - cnt;
+  const int incl = wave_scan(cnt), excl = incl - cnt;
   const int total = __builtin_amdgcn_readlane(incl, 63);
   for (int done = 0; done < total;) {
     const bool in = cnt > 0 && excl >= done && incl - done <= kCap;
@@ -331,21 +291,38 @@ __device__ __forceinline__ void walk_groups(const Rec &p, const Rec *__restrict_
     const int last = 63 - __builtin_clzll(__ballot(in));
     const int n = __builtin_amdgcn_readlane(incl, last) - done;
     done += n;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_fence();
     float acc[NA];
 #pragma unroll
     for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
-    for (int e0 = 0; e0 < n; e0 += 16) {
-      const unsigned e = list[min(e0 + (lane & 15), n - 1)];
-      const Rec q = Q[e & 0x7fffffffu];
-      unsigned first = (unsigned)__ballot((int)e < 0) & 0xffffu;
-      if (e0 == 0) first &= ~1u;  // the sums are 0
-      eval_rows<Rec, MODE, COMP, NA, 0>(p, q, first, n - e0, acc, dacc);
+    for (int e0 = 0; e0 < n; e0 += 64) {
+      const unsigned e = list[min(e0 + lane, n - 1)];
+      recs.put(lane, Q[e & 0x7fffffffu]);
+      unsigned long long first = __ballot((int)e < 0);
+      if (e0 == 0) first &= ~1ull;  // the sums are 0
+      wave_lds_fence();
+      const int m = min(64, n - e0);
+      int j = 0;
+      // records in flight: as many as the registers allow
+      constexpr int U = RecTraits<Rec>::FULL ? (RecTraits<Rec>::D == 3 ? 1 : 2) : MODE == kModeHess ? 2 : 4;
+      for (; j + U <= m; j += U) {
+        Rec q[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) q[k] = recs.get(j + k);
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+          if ((first >> (j + k)) & 1) flush_group<NA>(acc, dacc);
+          pair_eval<MODE, COMP>(p, q[k], acc);
+        }
+      }
+      for (; j < m; ++j) {
+        if ((first >> j) & 1) flush_group<NA>(acc, dacc);
+        pair_eval<MODE, COMP>(p, recs.get(j), acc);
+      }
+      wave_lds_fence();
     }
     flush_group<NA>(acc, dacc);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_fence();
   }
 }
 
@@ -448,10 +425,12 @@ __global__ __launch_bounds__(kNearBlock) __attribute__((amdgpu_waves_per_eu(MODE
                      : MODE == kModePose && !Tr::FULL ? 1 + D
                      : GRAD                           ? Tr::NACC
                                                       : 1;
-  // per wave kCap list entries, then the window's groups, 64 bits each; later
-  // the epilogue's staging
-  extern __shared__ unsigned s_dyn[];
-  unsigned *const s_bits = s_dyn + kNearWaves * kCap;
+  // per wave 64 records and kCap list entries, then the window's groups, 64
+  // bits each; later the epilogue's staging
+  using Recs = LdsRecs<Rec, COMP>;
+  extern __shared__ __attribute__((aligned(16))) unsigned s_dyn[];
+  unsigned *const s_list = s_dyn + kNearWaves * (sizeof(Recs) / 4);
+  unsigned *const s_bits = s_list + kNearWaves * kCap;
   __shared__ Rec s_p[64];
   __shared__ QBox s_row[kRows], s_quad[kQuads];
   int sb, qc;
@@ -460,6 +439,10 @@ __global__ __launch_bounds__(kNearBlock) __attribute__((amdgpu_waves_per_eu(MODE
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ppos = sb * 64 + lane;  // Hilbert position of the lane's point
   const bool valid = ppos < na.nP;
+  // the wave's first boxes, on their way while wave 0 prepares the stationary
+  // points: boxes are dealt to the waves one by one (near ones follow each other)
+  const int nbox = (na.nQ + 63) >> 6;
+  const QBox box0 = na.boxQ[min(wave + lane * kNearWaves, nbox - 1)];
 
   if (wave == 0) {
     const int pp = min(ppos, na.nP - 1);
@@ -499,20 +482,20 @@ __global__ __launch_bounds__(kNearBlock) __attribute__((amdgpu_waves_per_eu(MODE
 #pragma unroll
   for (int a = 0; a < kPosePart; ++a) r[a] = 0.0;
 
-  unsigned *const list = s_dyn + wave * kCap;
-  const int nbox = (na.nQ + 63) >> 6;
+  unsigned *const list = s_list + wave * kCap;
+  Recs &recs = reinterpret_cast<Recs *>(s_dyn)[wave];
   for (int w0 = 0; w0 < na.ngroups; w0 += na.win) {
     const int wn = min(na.win, na.ngroups - w0);
     if (w0 > 0) __syncthreads();  // the last window's bits have been read
     for (int i = threadIdx.x; i < 2 * wn; i += kNearBlock) s_bits[i] = 0u;
     __syncthreads();
     if (w0 == 0) p = s_p[lane];
-    // boxes are dealt to the waves one by one: near ones follow each other
     for (int b0 = wave; b0 < nbox; b0 += kNearBlock) {
       const int bl = b0 + lane * kNearWaves;
       bool hit = false;
       if (bl < nbox) {
-        const QBox q = na.boxQ[bl];
+        QBox q = box0;
+        if (b0 >= kNearBlock || w0 > 0) q = na.boxQ[bl];
 #pragma unroll
         for (int k = 0; k < kRows; ++k)
           hit = hit || box_near(s_row[k], q.lo[0], q.lo[1], q.lo[2], q.hi[0], q.hi[1], q.hi[2], q.lam);
@@ -549,7 +532,7 @@ __global__ __launch_bounds__(kNearBlock) __attribute__((amdgpu_waves_per_eu(MODE
         for (int gb = max(c * na.gpc, w0); gb < c1; gb += 64) {
           const int g = gb + lane;
           const bool own = g < c1;
-          walk_groups<Rec, MODE, COMP, NA>(p, Q, list, lane, own ? s_bits[2 * (g - w0)] : 0u,
+          walk_groups<Rec, MODE, COMP, NA>(p, Q, list, recs, lane, own ? s_bits[2 * (g - w0)] : 0u,
                                            own ? s_bits[2 * (g - w0) + 1] : 0u,
                                            c * na.qchunk + (g - c * na.gpc) * 64, dacc);
         }
@@ -562,7 +545,7 @@ __global__ __launch_bounds__(kNearBlock) __attribute__((amdgpu_waves_per_eu(MODE
         const int g = g0 + (lane * kNearWaves + wave) * na.qsplit + qc;
         const bool own = g < wn;
         const int c = (w0 + g) / na.gpc;
-        walk_groups<Rec, MODE, COMP, NA>(p, Q, list, lane, own ? s_bits[2 * g] : 0u, own ? s_bits[2 * g + 1] : 0u,
+        walk_groups<Rec, MODE, COMP, NA>(p, Q, list, recs, lane, own ? s_bits[2 * g] : 0u, own ? s_bits[2 * g + 1] : 0u,
                                          c * na.qchunk + (w0 + g - c * na.gpc) * 64, dacc);
       }
     }
@@ -805,7 +788,8 @@ static void launch_near_x(dugma_ctx *c, const Plan &pl, const Sets &st, const Po
                             : MODE == kModePoint ? sizeof(double) * kNearBlock * ((RecTraits<Rec>::NACC + 1) / 2)
                                                  : sizeof(double) * kNearBlock * kPosePart;
   const size_t lds =
-      std::max(kStage, sizeof(unsigned) * kNearWaves * kCap + (size_t)8 * std::min(pl.ngroups, kWinGroups));
+      std::max(kStage, kNearWaves * (sizeof(LdsRecs<Rec, COMP>) + sizeof(unsigned) * kCap) +
+                           (size_t)8 * std::min(pl.ngroups, kWinGroups));
   const void *P = XSRC ? (const void *)c->dSsrc : st.P;
   hipLaunchKernelGGL((k_near<Rec, MODE, COMP, XSRC>), tile_grid(pl.pblocks, pl.qsplit, na.xcd_map),
                      dim3(kNearBlock), lds, c->stream, P, (const Rec *)st.Q, na, ps, out, hess);

@@ -230,6 +230,100 @@ __device__ __forceinline__ void pair_eval(const Rec2I &p, const Rec2I &q, float 
 
 #undef DUGMA_DIFF
 
+// ---- streamed records through LDS -----------------------------------------
+// 64 streamed records of one wave: lane l puts record l, then every lane reads
+// the same one at a time (a wave-uniform address: broadcast, no bank conflict),
+// so that all operands of a pair are VGPRs (an add of two VGPRs issues in 2.5
+// cycles a wave, with an SGPR or DPP operand in 4.5).  Only the words that
+// pair_eval<., COMP> reads are held.  A batched pass over 17 G isotropic pairs
+// took 6.1 ms, with DPP row_newbcast operands 8.1, streamed through SGPRs
+// (consecutive records only) 5.4.
+__device__ __forceinline__ void wave_lds_fence() {  // orders a wave's own LDS writes and reads
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <class Rec, int COMP> struct LdsRecs;
+template <int COMP> struct LdsRecs<Rec3F, COMP> {
+  float4 a[64], b[64];
+  float c[64];
+  float4 l[COMP == 1 ? 64 : 1];
+  __device__ __forceinline__ void put(int i, const Rec3F &r) {
+    a[i] = make_float4(r.hx, r.hy, r.hz, r.s11);
+    b[i] = make_float4(r.s22, r.s33, r.s12, r.s13);
+    c[i] = r.s23;
+    if (COMP == 1) l[i] = make_float4(r.lx, r.ly, r.lz, 0.0f);
+  }
+  __device__ __forceinline__ Rec3F get(int i) const {
+    const float4 u = a[i], v = b[i];
+    Rec3F q;
+    q.hx = u.x; q.hy = u.y; q.hz = u.z; q.s11 = u.w;
+    q.s22 = v.x; q.s33 = v.y; q.s12 = v.z; q.s13 = v.w;
+    q.s23 = c[i];
+    if (COMP == 1) {
+      const float4 w = l[i];
+      q.lx = w.x; q.ly = w.y; q.lz = w.z;
+    }
+    return q;
+  }
+};
+template <int COMP> struct LdsRecs<Rec3I, COMP> {
+  float4 a[64], l[COMP == 1 ? 64 : 1];
+  __device__ __forceinline__ void put(int i, const Rec3I &r) {
+    a[i] = make_float4(r.hx, r.hy, r.hz, r.s);
+    if (COMP == 1) l[i] = make_float4(r.lx, r.ly, r.lz, 0.0f);
+  }
+  __device__ __forceinline__ Rec3I get(int i) const {
+    const float4 u = a[i];
+    Rec3I q;
+    q.hx = u.x; q.hy = u.y; q.hz = u.z; q.s = u.w;
+    if (COMP == 1) {
+      const float4 w = l[i];
+      q.lx = w.x; q.ly = w.y; q.lz = w.z;
+    }
+    return q;
+  }
+};
+template <int COMP> struct LdsRecs<Rec2F, COMP> {
+  float4 a[64];
+  float c[64];
+  float2 l[COMP == 1 ? 64 : 1];
+  __device__ __forceinline__ void put(int i, const Rec2F &r) {
+    a[i] = make_float4(r.hx, r.hy, r.s11, r.s12);
+    c[i] = r.s22;
+    if (COMP == 1) l[i] = make_float2(r.lx, r.ly);
+  }
+  __device__ __forceinline__ Rec2F get(int i) const {
+    const float4 u = a[i];
+    Rec2F q;
+    q.hx = u.x; q.hy = u.y; q.s11 = u.z; q.s12 = u.w;
+    q.s22 = c[i];
+    if (COMP == 1) {
+      const float2 w = l[i];
+      q.lx = w.x; q.ly = w.y;
+    }
+    return q;
+  }
+};
+template <int COMP> struct LdsRecs<Rec2I, COMP> {
+  float4 a[64];
+  float l[COMP == 1 ? 64 : 1];
+  __device__ __forceinline__ void put(int i, const Rec2I &r) {
+    a[i] = make_float4(r.hx, r.hy, r.s, r.lx);
+    if (COMP == 1) l[i] = r.ly;
+  }
+  __device__ __forceinline__ Rec2I get(int i) const {
+    const float4 u = a[i];
+    Rec2I q;
+    q.hx = u.x; q.hy = u.y; q.s = u.z;
+    if (COMP == 1) {
+      q.lx = u.w;
+      q.ly = l[i];
+    }
+    return q;
+  }
+};
+
 // ---- pose-gradient contribution of one stationary target ------------------
 // The energy is invariant under one rigid motion of both clouds, so the
 // gradient for moving the sources (rotation about t, then translation) is
