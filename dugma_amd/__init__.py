@@ -278,10 +278,11 @@ def energy_grad_points(h, R, t, cov="auto"):
     t = _cm(np.ravel(t))
     E = ctypes.c_double()
     gpose = np.zeros(6 if D == 3 else 3)
-    gX = np.zeros((N, D))
-    gXC = np.zeros((N, D, D))
-    gY = np.zeros((M, D))
-    gYC = np.zeros((M, D, D))
+    # written whole by the call
+    gX = np.empty((N, D))
+    gXC = np.empty((N, D, D))
+    gY = np.empty((M, D))
+    gYC = np.empty((M, D, D))
     gdT = np.zeros(12 if D == 3 else 4)
     _lib.check(_lib.load().dugma_energy_grad_points(h.ptr, _dp(R), _dp(t), _cov_mode(cov),
                                                     ctypes.byref(E), _dp(gpose), _dp(gX), _dp(gXC),

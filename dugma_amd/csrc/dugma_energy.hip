@@ -1074,7 +1074,142 @@ static void perturb(int D, const double *R, const double *t, const double *p,
   }
 }
 
-constexpr size_t kHostChunk = 4096;  // points per host task of the per-point conversion
+// Per-point gradients on the way out: from a point's sums (NACC of point_pass)
+// to the caller's units and layout -- gradient of the point (D) at P + i D, of
+// its covariance (D x D, column-major) at C + i D D, i its original index -- and,
+// per workgroup, kPointSums sums: [E, dE/dw (3) or dE/dtheta, dE/dt (3), dE/ddR
+// (9, column-major, at identity)], the pose's of the sources only.  FP64, one
+// thread per point; on the host (8 threads) the same took 1.3 ms for two
+// 76,800-point clouds, here 12 us.
+constexpr int kPointSums = 16;
+struct PointUnits {
+  double cn, gpos, gcov;  // Gaussian norm; unscaling of point and covariance gradients
+};
+template <int D, bool TARGET>
+__global__ __launch_bounds__(kBlock) void k_points_out(const double *__restrict__ acc,
+                                                       const double *__restrict__ src,
+                                                       const int *__restrict__ idx, int nP, PoseArg ps,
+                                                       PointUnits pu, double *__restrict__ P,
+                                                       double *__restrict__ C, double *__restrict__ sums) {
+  constexpr int DD = D * D, NACC = D == 3 ? kAcc3F : kAcc2F;
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  double s[kPointSums];
+#pragma unroll
+  for (int a = 0; a < kPointSums; ++a) s[a] = 0.0;
+  if (k < nP) {
+    double a[NACC];
+#pragma unroll
+    for (int q = 0; q < NACC; ++q) a[q] = acc[(size_t)k * NACC + q];
+    const size_t i = (size_t)idx[k];
+    double H[DD];  // dE/dS
+#pragma unroll
+    for (int u = 0; u < D; ++u)
+#pragma unroll
+      for (int v = u; v < D; ++v) {
+        const int q = 1 + D + (D == 3 ? (u == 0 ? v : u == 1 ? 2 + v : 5) : u + v);
+        H[u + D * v] = H[v + D * u] = 0.5 * pu.cn * a[q];
+      }
+    if constexpr (TARGET) {
+      s[0] = a[0];
+#pragma unroll
+      for (int d = 0; d < D; ++d) P[i * D + d] = -pu.cn * a[1 + d] * pu.gpos;
+#pragma unroll
+      for (int q = 0; q < DD; ++q) C[i * DD + q] = H[q] * pu.gcov;
+    } else {
+      const double *x = src + (size_t)k * (D + DD);
+      const double *R = ps.R;
+      double g[D], p[D], RS[DD], Sp[DD];
+#pragma unroll
+      for (int d = 0; d < D; ++d) g[d] = -pu.cn * a[1 + d];  // dE/dx'
+#pragma unroll
+      for (int d = 0; d < D; ++d) {  // R x (= x' - t)
+        double v = 0;
+#pragma unroll
+        for (int b = 0; b < D; ++b) v += R[d + D * b] * x[b];
+        p[d] = v;
+      }
+#pragma unroll
+      for (int u = 0; u < D; ++u)
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+          double v = 0;
+#pragma unroll
+          for (int b = 0; b < D; ++b) v += R[u + D * b] * x[D + b + D * c];
+          RS[u + D * c] = v;
+        }
+#pragma unroll
+      for (int u = 0; u < D; ++u)
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+          double v = 0;
+#pragma unroll
+          for (int b = 0; b < D; ++b) v += RS[u + D * b] * R[c + D * b];
+          Sp[u + D * c] = v;
+        }
+      double HS[DD], SH[DD];
+#pragma unroll
+      for (int u = 0; u < D; ++u)
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+          double v = 0, w = 0;
+#pragma unroll
+          for (int b = 0; b < D; ++b) {
+            v += H[u + D * b] * Sp[b + D * c];
+            w += Sp[u + D * b] * H[b + D * c];
+          }
+          HS[u + D * c] = v;
+          SH[u + D * c] = w;
+        }
+      if constexpr (D == 3) {  // p x g - 2 vee(S'H - HS')
+        s[1] = p[1] * g[2] - p[2] * g[1] - 2.0 * (SH[2 + 3 * 1] - HS[2 + 3 * 1]);
+        s[2] = p[2] * g[0] - p[0] * g[2] - 2.0 * (SH[0 + 3 * 2] - HS[0 + 3 * 2]);
+        s[3] = p[0] * g[1] - p[1] * g[0] - 2.0 * (SH[1 + 3 * 0] - HS[1 + 3 * 0]);
+      } else {  // tr(H (J S' - S' J)) = tr((S'H - HS') J) = 2 (S'H - HS')_12
+        s[1] = g[1] * p[0] - g[0] * p[1] + 2.0 * (SH[0 + 2 * 1] - HS[0 + 2 * 1]);
+      }
+#pragma unroll
+      for (int d = 0; d < D; ++d) s[4 + d] = g[d];
+      // dE/d dR at identity: g p^T + 2 H S'
+#pragma unroll
+      for (int u = 0; u < D; ++u)
+#pragma unroll
+        for (int c = 0; c < D; ++c) s[7 + u + D * c] = g[u] * p[c] + 2.0 * HS[u + D * c];
+#pragma unroll
+      for (int b = 0; b < D; ++b) {
+        double v = 0;
+#pragma unroll
+        for (int u = 0; u < D; ++u) v += R[u + D * b] * g[u];
+        P[i * D + b] = v * pu.gpos;
+      }
+#pragma unroll
+      for (int b = 0; b < D; ++b)
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+          double v = 0;
+#pragma unroll
+          for (int u = 0; u < D; ++u)
+#pragma unroll
+            for (int e = 0; e < D; ++e) v += R[u + D * b] * H[u + D * e] * R[e + D * c];
+          C[i * DD + b + D * c] = v * pu.gcov;
+        }
+    }
+  }
+  // workgroup sums in a fixed order
+  __shared__ double red[kBlock / 64][kPointSums];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int a = 0; a < (TARGET ? 1 : kPointSums); ++a) {
+    const double v = wave_sum(s[a]);
+    if (lane == 0) red[wave][a] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < (TARGET ? 1 : kPointSums)) {
+    double v = red[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; ++w) v += red[w][threadIdx.x];
+    sums[(size_t)blockIdx.x * kPointSums + threadIdx.x] = v;
+  }
+}
 
 // One per-point pass (stationary cloud st.stat), full covariance records;
 // writes per-point FP64 sums [nP][NACC] to out (device).
@@ -1287,167 +1422,84 @@ extern "C" int dugma_energy_grad_points(dugma_ctx *ctx, const double *R,
   if (rc) return rc;
   const Sets onT = {0, c->dTrecF, c->dSrecF, lam_scale}, onS = {1, c->dSrecF, c->dTrecF, lam_scale};
   const size_t nT = c->nT, nS = c->nS;
-  rc = c->scratch2.ensure(sizeof(double) * (nT + nS) * nacc);
-  if (rc) return rc;
-  double *acc = (double *)c->scratch2.ptr;
-  rc = c->hstage.ensure(sizeof(double) * (nT + nS) * nacc);
-  if (rc) return rc;
-  const double *hT = (const double *)c->hstage.ptr, *hS = hT + nT * nacc;
-  rc = refresh_host_sources(c);  // the host copy of the sources, before the passes (it may sync)
-  if (rc) return rc;
-  if (!c->evpts) DUGMA_HIP(hipEventCreateWithFlags(&c->evpts, hipEventDisableTiming));
-  // target pass, its sums on their way to the host, then the source pass:
-  // the host converts the target sums while the source pass runs
-  rc = point_pass(c, onT, ps, 1, acc);
-  hipError_t e = hipSuccess;
-  if (!rc) e = hipMemcpyAsync(c->hstage.ptr, acc, sizeof(double) * nT * nacc, hipMemcpyDeviceToHost, c->stream);
-  if (!rc && e == hipSuccess) e = hipEventRecord(c->evpts, c->stream);
-  if (!rc && e == hipSuccess) rc = point_pass(c, onS, ps, 2, acc + nT * nacc);
-  if (!rc && e == hipSuccess)
-    e = hipMemcpyAsync((double *)c->hstage.ptr + nT * nacc, acc + nT * nacc, sizeof(double) * nS * nacc,
-                       hipMemcpyDeviceToHost, c->stream);
-  clear_points();  // while the passes run
-  if (rc) return rc;
-  if (e == hipSuccess) e = hipEventSynchronize(c->evpts);
-  if (e != hipSuccess) return hip_fail(e, "dugma_energy_grad_points: download");
-
-  // Everything below is in scaled units until the final unscaling:
-  // positions x s, covariances x s^2, energy / s^D.
+  // Everything on the device is in scaled units: positions x s, covariances
+  // x s^2, energy / s^D.
   const double cn = gauss_norm(D);
   const double sc = c->scale, sD = std::pow(sc, D);
-  auto cov_grad = [&](const double *a, double *G) {
+  const double gpos = sD * sc;
+  const PointUnits pu = {cn, gpos, sD * sc * sc};
+  // device: the passes' sums | what goes to the host, targets | sources, each
+  // workgroup sums, then the points' gradients, then the covariances'
+  const size_t gridT = (nT + kBlock - 1) / kBlock, gridS = (nS + kBlock - 1) / kBlock;
+  const size_t lenT = gridT * kPointSums + (size_t)N * (D + DD), lenS = gridS * kPointSums + (size_t)M * (D + DD);
+  const size_t len_acc = (nT + nS) * nacc;
+  rc = c->scratch2.ensure(sizeof(double) * (len_acc + lenT + lenS));
+  if (rc) return rc;
+  rc = c->hstage.ensure(sizeof(double) * (lenT + lenS));
+  if (rc) return rc;
+  double *acc = (double *)c->scratch2.ptr;
+  double *dT = acc + len_acc, *dS = dT + lenT;
+  double *hT = (double *)c->hstage.ptr, *hS = hT + lenT;
+  if (!c->evpts) DUGMA_HIP(hipEventCreateWithFlags(&c->evpts, hipEventDisableTiming));
+  // Target pass, its results on their way to the host, then the source pass:
+  // the host hands the targets' gradients out while the source pass runs.
+  // Points left out keep zero gradients.
+  auto out = [&](bool tgt) -> int {
+    const size_t n = tgt ? nT : nS, all = tgt ? N : M, grid = tgt ? gridT : gridS, len = tgt ? lenT : lenS;
+    double *sums = tgt ? dT : dS, *P = sums + grid * kPointSums, *C = P + all * D;
+    if (n < all) DUGMA_HIP(hipMemsetAsync(P, 0, sizeof(double) * all * (D + DD), c->stream));
+    const double *a = tgt ? acc : acc + nT * nacc;
+    const int *idx = tgt ? c->dTidx : c->dSidx;
+#define POINTS_OUT(DD_, TT)                                                                                \
+  hipLaunchKernelGGL((k_points_out<DD_, TT>), dim3((unsigned)grid), dim3(kBlock), 0, c->stream, a, c->dSsrc, idx, \
+                     (int)n, ps, pu, P, C, sums)
     if (D == 3) {
-      static const int ij[6][2] = {{0, 0}, {0, 1}, {0, 2}, {1, 1}, {1, 2}, {2, 2}};
-      for (int k = 0; k < 6; ++k) {
-        double v = 0.5 * cn * a[4 + k];
-        G[ij[k][0] + 3 * ij[k][1]] = v;
-        G[ij[k][1] + 3 * ij[k][0]] = v;
-      }
+      if (tgt) POINTS_OUT(3, true); else POINTS_OUT(3, false);
     } else {
-      static const int ij[3][2] = {{0, 0}, {0, 1}, {1, 1}};
-      for (int k = 0; k < 3; ++k) {
-        double v = 0.5 * cn * a[3 + k];
-        G[ij[k][0] + 2 * ij[k][1]] = v;
-        G[ij[k][1] + 2 * ij[k][0]] = v;
-      }
+      if (tgt) POINTS_OUT(2, true); else POINTS_OUT(2, false);
     }
+#undef POINTS_OUT
+    DUGMA_HIP(hipGetLastError());
+    const bool points = tgt ? (gX || gXC) : (gY || gYC);
+    DUGMA_HIP(hipMemcpyAsync(tgt ? hT : hS, sums, sizeof(double) * (points ? len : grid * kPointSums),
+                             hipMemcpyDeviceToHost, c->stream));
+    return DUGMA_OK;
   };
-  const double gpos = sD * sc, gcov = sD * sc * sc;  // unscaling of point / covariance gradients
-  // Per-point results go to the caller's arrays from worker threads, over
-  // fixed chunks of points; the energy and pose sums of each chunk are then
-  // added in chunk order, so results do not depend on the thread count.
-  struct PoseSums {
-    double gw[3] = {0, 0, 0}, gt[3] = {0, 0, 0}, gth = 0.0, G[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  rc = point_pass(c, onT, ps, 1, acc);
+  if (!rc) rc = out(true);
+  if (rc) return rc;
+  hipError_t e = hipEventRecord(c->evpts, c->stream);
+  if (e != hipSuccess) return hip_fail(e, "dugma_energy_grad_points: event");
+  rc = point_pass(c, onS, ps, 2, acc + nT * nacc);
+  if (!rc) rc = out(false);
+  if (rc) return rc;
+  // the caller's arrays, in pieces, on a few threads (fresh pages are touched
+  // here for the first time: a serial fill of them took 2 ms)
+  auto hand_out = [&](const double *P, size_t all, double *gP, double *gC) {
+    const size_t np = gP ? all * D : 0, nc = gC ? all * DD : 0;
+    const double *C = P + all * D;
+    constexpr size_t kPiece = size_t(1) << 16;  // 512 KiB
+    const size_t kp = (np + kPiece - 1) / kPiece, kc = (nc + kPiece - 1) / kPiece;
+    parallel_for(kp + kc, [&](size_t q) {
+      const size_t o = (q < kp ? q : q - kp) * kPiece;
+      if (q < kp)
+        memcpy(gP + o, P + o, sizeof(double) * std::min(kPiece, np - o));
+      else
+        memcpy(gC + o, C + o, sizeof(double) * std::min(kPiece, nc - o));
+    });
   };
-  auto target_chunk = [&](size_t k0, size_t k1, double &Epart) {
-    double e = 0.0;
-    for (size_t k = k0; k < k1; ++k) {
-      const double *a = hT + k * nacc;
-      e += a[0];
-      const int i = c->hTidx[k];
-      if (gX)
-        for (int d = 0; d < D; ++d) gX[(size_t)i * D + d] = -cn * a[1 + d] * gpos;
-      if (gXC) {
-        double G[9];
-        cov_grad(a, G);
-        for (int q = 0; q < DD; ++q) gXC[(size_t)i * DD + q] = G[q] * gcov;
-      }
-    }
-    Epart = e;
-  };
-  auto source_chunk = [&](size_t k0, size_t k1, PoseSums &P) {
-    for (size_t k = k0; k < k1; ++k) {
-      const double *a = hS + k * nacc;
-      const double *s = c->hSsrc.data() + k * (D + DD);
-      double g[3], H[9], p[3], Sp[9];
-      for (int d = 0; d < D; ++d) g[d] = -cn * a[1 + d];  // dE/dx'_j
-      cov_grad(a, H);                                     // dE/dS'_j
-      for (int d = 0; d < D; ++d) {
-        double v = 0;
-        for (int b = 0; b < D; ++b) v += R[d + D * b] * s[b];
-        p[d] = v;  // R x_j  (= x'_j - t)
-      }
-      double RS[9];
-      for (int a1 = 0; a1 < D; ++a1)
-        for (int c1 = 0; c1 < D; ++c1) {
-          double v = 0;
-          for (int b = 0; b < D; ++b) v += R[a1 + D * b] * s[D + b + D * c1];
-          RS[a1 + D * c1] = v;
-        }
-      for (int a1 = 0; a1 < D; ++a1)
-        for (int c1 = 0; c1 < D; ++c1) {
-          double v = 0;
-          for (int b = 0; b < D; ++b) v += RS[a1 + D * b] * R[c1 + D * b];
-          Sp[a1 + D * c1] = v;
-        }
-      for (int d = 0; d < D; ++d) P.gt[d] += g[d];
-      double HS[9], SH[9];
-      for (int a1 = 0; a1 < D; ++a1)
-        for (int c1 = 0; c1 < D; ++c1) {
-          double v = 0, w = 0;
-          for (int b = 0; b < D; ++b) {
-            v += H[a1 + D * b] * Sp[b + D * c1];
-            w += Sp[a1 + D * b] * H[b + D * c1];
-          }
-          HS[a1 + D * c1] = v;
-          SH[a1 + D * c1] = w;
-        }
-      // dE/d dR at identity: g p^T + 2 H S'
-      for (int a1 = 0; a1 < D; ++a1)
-        for (int c1 = 0; c1 < D; ++c1) P.G[a1 + D * c1] += g[a1] * p[c1] + 2.0 * HS[a1 + D * c1];
-      if (D == 3) {
-        P.gw[0] += p[1] * g[2] - p[2] * g[1];
-        P.gw[1] += p[2] * g[0] - p[0] * g[2];
-        P.gw[2] += p[0] * g[1] - p[1] * g[0];
-        // -2 vee(S'H - HS')
-        P.gw[0] -= 2.0 * (SH[2 + 3 * 1] - HS[2 + 3 * 1]);
-        P.gw[1] -= 2.0 * (SH[0 + 3 * 2] - HS[0 + 3 * 2]);
-        P.gw[2] -= 2.0 * (SH[1 + 3 * 0] - HS[1 + 3 * 0]);
-      } else {
-        P.gth += g[1] * p[0] - g[0] * p[1];
-        // tr(H (J S' - S' J)) = tr((S'H - HS') J) = 2 (S'H - HS')_12
-        P.gth += 2.0 * (SH[0 + 2 * 1] - HS[0 + 2 * 1]);
-      }
-      const int j = c->hSidx[k];
-      if (gY)
-        for (int b = 0; b < D; ++b) {
-          double v = 0;
-          for (int a1 = 0; a1 < D; ++a1) v += R[a1 + D * b] * g[a1];
-          gY[(size_t)j * D + b] = v * gpos;
-        }
-      if (gYC) {
-        double *o = gYC + (size_t)j * DD;
-        for (int b = 0; b < D; ++b)
-          for (int c1 = 0; c1 < D; ++c1) {
-            double v = 0;
-            for (int a1 = 0; a1 < D; ++a1)
-              for (int e = 0; e < D; ++e) v += R[a1 + D * b] * H[a1 + D * e] * R[e + D * c1];
-            o[b + D * c1] = v * gcov;
-          }
-      }
-    }
-  };
-  const size_t ncT = (nT + kHostChunk - 1) / kHostChunk, ncS = (nS + kHostChunk - 1) / kHostChunk;
-  std::vector<double> Epart(ncT);
-  std::vector<PoseSums> Ppart(ncS);
-  parallel_for(ncT, [&](size_t q) { target_chunk(q * kHostChunk, std::min(nT, (q + 1) * kHostChunk), Epart[q]); });
-  e = hipStreamSynchronize(c->stream);  // the source pass and its sums
+  e = hipEventSynchronize(c->evpts);
   if (e != hipSuccess) return hip_fail(e, "dugma_energy_grad_points: download");
-  parallel_for(ncS, [&](size_t q) {
-    source_chunk(q * kHostChunk, std::min(nS, (q + 1) * kHostChunk), Ppart[q]);
-  });
-  double Etot = 0.0;
-  for (double e : Epart) Etot += e;
+  hand_out(hT + gridT * kPointSums, N, gX, gXC);
+  e = hipStreamSynchronize(c->stream);  // the source pass and its results
+  if (e != hipSuccess) return hip_fail(e, "dugma_energy_grad_points: download");
+  hand_out(hS + gridS * kPointSums, M, gY, gYC);
+  double Etot = 0.0, ps_sum[kPointSums] = {0.0};
+  for (size_t q = 0; q < gridT; ++q) Etot += hT[q * kPointSums];
+  for (size_t q = 0; q < gridS; ++q)
+    for (int a = 1; a < kPointSums; ++a) ps_sum[a] += hS[q * kPointSums + a];
   if (E) *E = cn * Etot * sD;
-  double gw[3] = {0, 0, 0}, gt[3] = {0, 0, 0}, gth = 0.0, G[9] = {0};
-  for (const PoseSums &P : Ppart) {
-    for (int a = 0; a < 3; ++a) {
-      gw[a] += P.gw[a];
-      gt[a] += P.gt[a];
-    }
-    gth += P.gth;
-    for (int q = 0; q < 9; ++q) G[q] += P.G[q];
-  }
+  const double *gw = ps_sum + 1, gth = ps_sum[1], *gt = ps_sum + 4, *G = ps_sum + 7;
   // unscale: rotation / dR parts ~ s^D, translation parts ~ s^(D+1)
   if (gpose) {
     if (D == 3) {
