@@ -261,12 +261,11 @@ using namespace dugma;
 
 static void free_ctx(dugma_ctx *c) {
   if (!c) return;
-  void *ptrs[] = {c->dX, c->dXCinv, c->dY, c->dYCinv, c->dgX, c->dgY,
-                  c->dTidx, c->dSidx, c->dTrecF, c->dTrecI, c->dSsrc,
-                  c->dSrecF, c->dSrecI};
+  void *ptrs[] = {c->dX, c->dXCinv, c->dY, c->dYCinv, c->dgX, c->dgY};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
-  c->nearbuf.release();
+  c->energybuf.release();
+  c->isobuf.release();
   c->part.release();
   c->scratch2.release();
   c->sigbuf.release();
@@ -425,14 +424,28 @@ extern "C" int dugma_init(const double *X, const double *X_C, const double *Y,
     make_target_records(D, keepT, X, X_C, sc, recF, recI, c->iso);
     const size_t recsz = (D == 3) ? sizeof(Rec3F) : sizeof(Rec2F);
     const size_t recszI = (D == 3) ? sizeof(Rec3I) : sizeof(Rec2I);
-    const size_t nTa = (size_t)std::max(c->nT, 1), nSa = (size_t)std::max(c->nS, 1);
-    TRY(dmalloc(&c->dTidx, nTa));
-    TRY(dmalloc(&c->dSidx, nSa));
-    TRY(dmalloc((char **)&c->dTrecF, nTa * recsz));
-    TRY(dmalloc((char **)&c->dSrecF, nSa * recsz));
-    if (c->iso) {
-      TRY(dmalloc((char **)&c->dTrecI, nTa * recszI));
-      TRY(dmalloc((char **)&c->dSrecI, nSa * recszI));
+    // one allocation for all that the energy passes read (a first pass on a
+    // new context then misses the TLB once, not per array)
+    {
+      const size_t nT = c->nT, nS = c->nS;
+      struct Part {
+        void **p;
+        size_t bytes;
+      } parts[] = {{(void **)&c->dTidx, nT * sizeof(int)},    {(void **)&c->dSidx, nS * sizeof(int)},
+                   {&c->dTrecF, nT * recsz},                  {&c->dSrecF, nS * recsz},
+                   {&c->dTrecI, c->iso ? nT * recszI : 0},    {&c->dSrecI, c->iso ? nS * recszI : 0},
+                   {(void **)&c->dSsrc, nS * (D + DD) * sizeof(double)}};
+      const size_t near = near_bytes(c->nT, c->nS);
+      size_t total = near;
+      for (const Part &q : parts) total += (q.bytes + 255) & ~(size_t)255;
+      TRY(c->energybuf.ensure(total));
+      char *at = (char *)c->energybuf.ptr;
+      near_place(c, at);
+      at += near;
+      for (const Part &q : parts) {
+        *q.p = q.bytes ? at : nullptr;
+        at += (q.bytes + 255) & ~(size_t)255;
+      }
     }
     // source data: FP32-rounded point (D) then symmetric covariance (D*D)
     // per kept point, scaled, held in FP64 for the per-call transform
@@ -445,7 +458,6 @@ extern "C" int dugma_init(const double *X, const double *X_C, const double *Y,
       for (int a = 0; a < D; ++a)
         for (int b = 0; b < D; ++b) o[D + a + D * b] = sym32(S, D, a, b) * sc2;
     }
-    TRY(dmalloc(&c->dSsrc, std::max<size_t>(src.size(), 1)));
     hipError_t e3 = hipSuccess;
     if (c->nT > 0) {
       e3 = hipMemcpy(c->dTidx, keepT.data(), sizeof(int) * c->nT, hipMemcpyHostToDevice);

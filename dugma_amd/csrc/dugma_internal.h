@@ -254,7 +254,8 @@ struct dugma_ctx {
   long long pair_launches = 0;
 
   dugma::NearCloud near[2];  // spatial index: targets, sources
-  dugma::DevBuf nearbuf;     // its arrays
+  dugma::DevBuf energybuf;   // kept-point lists, records, source data and the index
+  dugma::DevBuf isobuf;      // isotropic records of a context that became isotropic
 
   dugma::DevBuf part;        // pair-kernel partials
   dugma::DevBuf scratch2;    // reductions / k-NN merge

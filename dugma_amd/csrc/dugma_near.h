@@ -72,6 +72,9 @@ __device__ __forceinline__ float quad_max(float v) {
   return fmaxf(v, dpp_f<0x4E>(v));
 }
 
+// The index's arrays: their size, and where they lie.
+size_t near_bytes(int nT, int nS);
+void near_place(dugma_ctx *c, char *base);
 // Hilbert order of both clouds (init): lo, hi are the kept points' bounds.
 int near_build(dugma_ctx *c, const double lo[2][3], const double hi[2][3]);
 // lam, aux and boxes again after covariances changed on the device; cloud 0

@@ -220,27 +220,40 @@ int near_index_sources(dugma_ctx *c, bool iso, const void *recs, float lam_scale
   return DUGMA_OK;
 }
 
+static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+size_t near_bytes(int nT, int nS) {
+  size_t bytes = 0;
+  for (const size_t m : {(size_t)nT, (size_t)nS})
+    bytes += al256(m * sizeof(int)) + al256(m * sizeof(QAux)) + al256((m + 63) / 64 * sizeof(QBox)) +
+             al256(m * sizeof(float));
+  return bytes;
+}
+
+void near_place(dugma_ctx *c, char *b) {
+  for (int w = 0; w < 2; ++w) {
+    NearCloud &nc = c->near[w];
+    const size_t m = w == 0 ? c->nT : c->nS;
+    nc.ord = (int *)b;
+    b += al256(m * sizeof(int));
+    nc.aux = (QAux *)b;
+    b += al256(m * sizeof(QAux));
+    nc.box = (QBox *)b;
+    b += al256((m + 63) / 64 * sizeof(QBox));
+    nc.lam = (float *)b;
+    b += al256(m * sizeof(float));
+  }
+}
+
 int near_build(dugma_ctx *c, const double lo[2][3], const double hi[2][3]) {
   const int n[2] = {c->nT, c->nS};
   const int nmax = std::max(n[0], n[1]);
   if (nmax == 0) return DUGMA_OK;
-  auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  // one allocation for both clouds' arrays
-  size_t off[2][4], bytes = 0;
-  for (int w = 0; w < 2; ++w) {
-    const size_t m = (size_t)n[w], nb = (m + 63) / 64;
-    off[w][0] = bytes; bytes += al(m * sizeof(int));
-    off[w][1] = bytes; bytes += al(m * sizeof(QAux));
-    off[w][2] = bytes; bytes += al(nb * sizeof(QBox));
-    off[w][3] = bytes; bytes += al(m * sizeof(float));
-  }
-  int rc = c->nearbuf.ensure(bytes);
-  if (rc) return rc;
   size_t tmp = 0;
   DUGMA_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, (const unsigned *)nullptr, (unsigned *)nullptr,
                                                (const int *)nullptr, (int *)nullptr, nmax, 0, 30, c->stream));
-  const size_t bk = al((size_t)nmax * 4);
-  rc = c->scratch2.ensure(3 * bk + tmp);
+  const size_t bk = al256((size_t)nmax * 4);
+  int rc = c->scratch2.ensure(3 * bk + tmp);
   if (rc) return rc;
   char *sb = (char *)c->scratch2.ptr;
   unsigned *k0 = (unsigned *)sb, *k1 = (unsigned *)(sb + bk);
@@ -249,11 +262,6 @@ int near_build(dugma_ctx *c, const double lo[2][3], const double hi[2][3]) {
   const int D = c->D;
   for (int w = 0; w < 2; ++w) {
     NearCloud &nc = c->near[w];
-    char *b = (char *)c->nearbuf.ptr;
-    nc.ord = (int *)(b + off[w][0]);
-    nc.aux = (QAux *)(b + off[w][1]);
-    nc.box = (QBox *)(b + off[w][2]);
-    nc.lam = (float *)(b + off[w][3]);
     if (n[w] == 0) continue;
     // cubic cells over the largest extent
     double ext = 0.0;

@@ -1186,8 +1186,13 @@ extern "C" int dugma_update_sigma_knn(dugma_ctx *ctx, int which, int k, float *s
   if (c->iso && !was_iso) {
     // the context has just become isotropic: its isotropic records
     const size_t recszI = D == 3 ? sizeof(Rec3I) : sizeof(Rec2I);
-    if (!c->dTrecI) DUGMA_HIP(hipMalloc(&c->dTrecI, (size_t)c->nT * recszI));
-    if (!c->dSrecI) DUGMA_HIP(hipMalloc(&c->dSrecI, (size_t)c->nS * recszI));
+    if (!c->dTrecI) {
+      const size_t bT = al((size_t)c->nT * recszI);
+      rc = c->isobuf.ensure(bT + (size_t)c->nS * recszI);
+      if (rc) return rc;
+      c->dTrecI = c->isobuf.ptr;
+      c->dSrecI = (char *)c->isobuf.ptr + bT;
+    }
     const dim3 grid((c->nT + kSBlock - 1) / kSBlock);
     if (D == 3)
       hipLaunchKernelGGL(k_iso_records<3>, grid, blk, 0, c->stream, c->dTrecF, c->nT, c->dTrecI);
