@@ -54,11 +54,33 @@ __device__ __forceinline__ unsigned f2u_rn(float s) {
   return (unsigned)rintf(s);
 }
 
+// fl32(fl32(s2 / D) * 1e6) to the nearest u32 (update_sig.cu:255-263).
+template <int D>
+__device__ __forceinline__ unsigned quantise(float s2) {
+  // fl32(s2 / D): for D = 3 the FMA-corrected product below is the IEEE
+  // quotient for every non-negative finite float (checked exhaustively on
+  // the CPU by tests/arith/div3_exhaustive.c); for D = 2 halving is exact
+  constexpr float kThird = 1.0f / 3.0f;
+  float s;
+  if (D == 3 && s2 < __builtin_huge_valf()) {
+    const float q = s2 * kThird;
+    s = fmaf(fmaf(-3.0f, q, s2), kThird, q);
+  } else {
+    s = s2 * 0.5f;  // infinite and NaN stay what they are
+  }
+  return f2u_rn(s * 1000000.0f);
+}
+
 // update_sig.cu:238-265: per target the minimum over a chunk of sources of
 // rn_u32(fl32(fl32(|n - m|^2) / D) * 1e6), merged with atomicMin (the
 // minimum does not depend on the order).  IEEE FP32 semantics in source
 // order; the reference's binaries use -use_fast_math (compile.m:2), whose
-// division may differ in the last bit.
+// division may differ in the last bit.  The quantisation is monotone in
+// |n - m|^2, so the smallest is quantised once; a NaN, which quantises to 0, shows
+// in the largest bits.  Bound by FP32 issue: 10 operations a pair, 6,000 x
+// 6,000 in 11 us, 8 candidates' scalar loads at a time (24 us with every pair
+// quantised and one candidate ahead: the compiler folded that prefetch away and
+// each pair waited for its load); 20,000 x 15,000 206 -> 87 us a call.
 template <int D>
 __global__ __launch_bounds__(kSBlock) void k_nn1_quant(
     const float *__restrict__ X, int N, const float *__restrict__ Mp, int M,
@@ -70,37 +92,40 @@ __global__ __launch_bounds__(kSBlock) void k_nn1_quant(
   float n[3];
 #pragma unroll
   for (int a = 0; a < D; ++a) n[a] = X[(size_t)ii * D + a];
-  constexpr float kThird = 1.0f / 3.0f;
-  unsigned best = 4000000000u;
-  // candidate j + 1 is requested before candidate j is used (j0 < j1 for
-  // every workgroup; index clamped to the chunk)
-  float mn[3] = {Mp[(size_t)j0 * D], Mp[(size_t)j0 * D + 1], D == 3 ? Mp[(size_t)j0 * D + (D - 1)] : 0.0f};
-  for (int j = j0; j < j1; ++j) {
-    const float m[3] = {mn[0], mn[1], mn[2]};
-    const size_t jn = (size_t)min(j + 1, j1 - 1) * D;
-    mn[0] = Mp[jn];
-    mn[1] = Mp[jn + 1];
-    if (D == 3) mn[2] = Mp[jn + (D - 1)];
+  // squared distances as bits: non-negative floats order like unsigned, NaNs
+  // above them
+  unsigned lo = 0xffffffffu, hi = 0u;
+  auto pair = [&](const float *m) {
     const float e0 = n[0] - m[0], e1 = n[1] - m[1];
     float s2 = e0 * e0 + e1 * e1;
     if (D == 3) {
-      const float e2 = n[2] - m[2];
+      const float e2 = n[D - 1] - m[D - 1];
       s2 = s2 + e2 * e2;
     }
-    // fl32(s2 / D): for D = 3 the FMA-corrected product below is the IEEE
-    // quotient for every non-negative finite float (checked exhaustively on
-    // the CPU by tests/arith/div3_exhaustive.c); for D = 2 halving is exact
-    float s;
-    if (D == 3) {
-      const float q = s2 * kThird;
-      s = fmaf(fmaf(-3.0f, q, s2), kThird, q);
-    } else {
-      s = s2 * 0.5f;
-    }
-    s = s * 1000000.0f;
-    best = min(best, f2u_rn(s));
+    const unsigned b = __float_as_uint(s2);
+    lo = min(lo, b);
+    hi = max(hi, b);
+  };
+  // 8 candidates a step, the next 8 requested before these are used
+  constexpr int U = 8;
+  const float *c = Mp + (size_t)j0 * D;
+  float nx[U * D];
+  const int steps = (j1 - j0) / U;
+#pragma unroll
+  for (int q = 0; q < U * D; ++q) nx[q] = steps > 0 ? c[q] : 0.0f;
+  for (int s = 0; s < steps; ++s) {
+    float m[U * D];
+#pragma unroll
+    for (int q = 0; q < U * D; ++q) m[q] = nx[q];
+    c += s + 1 < steps ? U * D : 0;
+#pragma unroll
+    for (int q = 0; q < U * D; ++q) nx[q] = c[q];
+#pragma unroll
+    for (int k = 0; k < U; ++k) pair(m + k * D);
   }
-  if (i < N) atomicMin(qmin + i, best);
+  for (int j = j0 + steps * U; j < j1; ++j) pair(Mp + (size_t)j * D);
+  if (i >= N) return;
+  atomicMin(qmin + i, hi > 0x7f800000u ? 0u : min(4000000000u, quantise<D>(__uint_as_float(lo))));
 }
 
 // update_sig.cu:79-91 then 291-307 with n_c = 1: a[i] = fl32(q[i]) / 1e6
