@@ -253,9 +253,14 @@ int near_build(dugma_ctx *c, const double lo[2][3], const double hi[2][3]) {
   DUGMA_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, (const unsigned *)nullptr, (unsigned *)nullptr,
                                                (const int *)nullptr, (int *)nullptr, nmax, 0, 30, c->stream));
   const size_t bk = al256((size_t)nmax * 4);
-  int rc = c->scratch2.ensure(3 * bk + tmp);
+  // not the context's scratch: growing that in the first call would cost it a
+  // free (55 us)
+  struct Temp : DevBuf {
+    ~Temp() { release(); }
+  } temp;
+  int rc = temp.ensure(3 * bk + tmp);
   if (rc) return rc;
-  char *sb = (char *)c->scratch2.ptr;
+  char *sb = (char *)temp.ptr;
   unsigned *k0 = (unsigned *)sb, *k1 = (unsigned *)(sb + bk);
   int *v0 = (int *)(sb + 2 * bk);
   void *st = sb + 3 * bk;
@@ -284,6 +289,7 @@ int near_build(dugma_ctx *c, const double lo[2][3], const double hi[2][3]) {
     rc = near_refresh(c, w);
     if (rc) return rc;
   }
+  DUGMA_HIP(hipStreamSynchronize(c->stream));  // the sort's memory goes
   return DUGMA_OK;
 }
 

@@ -443,6 +443,19 @@ __device__ __forceinline__ int grid_cell(const float *x, const GridParams &g) {
   return (cz * g.ny + cy) * g.nx + cx;
 }
 
+// The key of a point: its cell, or the number of cells if a coordinate is not
+// finite (no candidate; as a query, answered without a search).
+template <int D>
+__device__ __forceinline__ int point_key(const float *__restrict__ P, int i, const GridParams &g, float *x) {
+  bool fin = true;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    x[a] = P[(size_t)i * D + a];
+    fin = fin && isfinite(x[a]);
+  }
+  return fin ? grid_cell<D>(x, g) : g.nx * g.ny * g.nz;
+}
+
 template <int D>
 __global__ __launch_bounds__(kSBlock) void k_grid_count(const float *__restrict__ P, int np,
                                                         const GridParams *__restrict__ gp,
@@ -450,65 +463,40 @@ __global__ __launch_bounds__(kSBlock) void k_grid_count(const float *__restrict_
   const int j = blockIdx.x * kSBlock + threadIdx.x;
   if (j >= np) return;
   float x[D];
-  bool fin = true;
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    x[a] = P[(size_t)j * D + a];
-    fin = fin && isfinite(x[a]);
-  }
-  if (!fin) return;
-  atomicAdd(cnt + grid_cell<D>(x, *gp), 1);
+  atomicAdd(cnt + point_key<D>(P, j, *gp, x), 1);
 }
 
-// Candidates into cell order (order inside a cell is arbitrary: the lists
-// are kept in (distance, index) order).  cnt counts down to 0.
+// Candidates into key order (order inside a cell is arbitrary: the lists
+// are kept in (distance, index) order), one 16-byte record each: coordinates and
+// index; those that are not finite lie behind the others.  cnt counts down to 0.
+// sidx (optional): the indices alone, the order of the queries where they are
+// the same points.
 template <int D>
 __global__ __launch_bounds__(kSBlock) void k_grid_scatter(const float *__restrict__ P, int np,
                                                           const GridParams *__restrict__ gp,
                                                           const int *__restrict__ start,
-                                                          int *__restrict__ cnt, float *__restrict__ spts,
+                                                          int *__restrict__ cnt, float4 *__restrict__ spts,
                                                           int *__restrict__ sidx) {
   const int j = blockIdx.x * kSBlock + threadIdx.x;
   if (j >= np) return;
   float x[D];
-  bool fin = true;
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    x[a] = P[(size_t)j * D + a];
-    fin = fin && isfinite(x[a]);
-  }
-  if (!fin) return;
-  const int cell = grid_cell<D>(x, *gp);
-  const int pos = start[cell] + atomicSub(cnt + cell, 1) - 1;
-#pragma unroll
-  for (int a = 0; a < D; ++a) spts[(size_t)pos * D + a] = x[a];
-  sidx[pos] = j;
+  const int key = point_key<D>(P, j, *gp, x);
+  const int pos = start[key] + atomicSub(cnt + key, 1) - 1;
+  spts[pos] = make_float4(x[0], x[1], D == 3 ? x[D - 1] : 0.0f, __int_as_float(j));
+  if (sidx) sidx[pos] = j;
 }
 
-// Queries into cell order too, so that the lanes of a wave search
-// neighbouring cells (shared ring extents, nearby candidate loads).  The key
-// is the query's cell, or the number of cells for a query with a
-// non-finite coordinate (answered without a search).  Each query's result
-// does not depend on the order.
-template <int D>
-__device__ __forceinline__ int query_key(const float *__restrict__ Q, int i, const GridParams &g) {
-  float x[D];
-  bool fin = true;
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    x[a] = Q[(size_t)i * D + a];
-    fin = fin && isfinite(x[a]);
-  }
-  return fin ? grid_cell<D>(x, g) : g.nx * g.ny * g.nz;
-}
-
+// Other queries go into key order too, so that the lanes of a wave search
+// neighbouring cells (shared ring extents, nearby candidate loads).  Each
+// query's result does not depend on the order.
 template <int D>
 __global__ __launch_bounds__(kSBlock) void k_query_count(const float *__restrict__ Q, int nq,
                                                          const GridParams *__restrict__ gp,
                                                          int *__restrict__ cnt) {
   const int i = blockIdx.x * kSBlock + threadIdx.x;
   if (i >= nq) return;
-  atomicAdd(cnt + query_key<D>(Q, i, *gp), 1);
+  float x[D];
+  atomicAdd(cnt + point_key<D>(Q, i, *gp, x), 1);
 }
 
 template <int D>
@@ -518,7 +506,8 @@ __global__ __launch_bounds__(kSBlock) void k_query_scatter(const float *__restri
                                                            int *__restrict__ cnt, int *__restrict__ qord) {
   const int i = blockIdx.x * kSBlock + threadIdx.x;
   if (i >= nq) return;
-  const int key = query_key<D>(Q, i, *gp);
+  float x[D];
+  const int key = point_key<D>(Q, i, *gp, x);
   qord[start[key] + atomicSub(cnt + key, 1) - 1] = i;
 }
 
@@ -543,23 +532,25 @@ __device__ __forceinline__ void topk_insert_lex(float *bd, int *bi, float dd, in
 }
 
 template <int D, int K>
-__device__ __forceinline__ void grid_visit(const float *q, int i, int self_exclude, int p0, int p1,
-                                           const float *__restrict__ spts, const int *__restrict__ sidx,
-                                           float *bd, int *bi) {
-  for (int pos = p0; pos < p1; ++pos) {
-    const int j = sidx[pos];
-    const float *p = spts + (size_t)pos * D;
-    const float dx = q[0] - p[0], dy = q[1] - p[1];
-    float dd;
-    if (D == 3) {
-      const float dz = q[2] - p[2];
-      dd = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-    } else {
-      dd = fmaf(dy, dy, dx * dx);
-    }
-    if (self_exclude && j == i) continue;
-    topk_insert_lex<K>(bd, bi, dd, j);
+__device__ __forceinline__ void grid_candidate(const float *q, int i, int self_exclude, const float4 p, float *bd,
+                                               int *bi) {
+  const int j = __float_as_int(p.w);
+  const float dx = q[0] - p.x, dy = q[1] - p.y;
+  float dd;
+  if (D == 3) {
+    const float dz = q[D - 1] - p.z;
+    dd = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+  } else {
+    dd = fmaf(dy, dy, dx * dx);
   }
+  if (self_exclude && j == i) return;
+  topk_insert_lex<K>(bd, bi, dd, j);
+}
+
+template <int D, int K>
+__device__ __forceinline__ void grid_visit(const float *q, int i, int self_exclude, int p0, int p1,
+                                           const float4 *__restrict__ spts, float *bd, int *bi) {
+  for (int pos = p0; pos < p1; ++pos) grid_candidate<D, K>(q, i, self_exclude, spts[pos], bd, bi);
 }
 
 // Lower bound of the squared distance from q to every cell outside the
@@ -601,9 +592,10 @@ __device__ __forceinline__ double unvisited_dist2(const float *q, int cx, int cy
 
 template <int D, int K>
 __global__ __launch_bounds__(kSBlock) void k_knn_grid(
-    const float *__restrict__ Q, int nq, const int *__restrict__ qord, const float *__restrict__ spts,
-    const int *__restrict__ sidx, const int *__restrict__ start, const GridParams *__restrict__ gp,
+    const float *__restrict__ Q, int nq, const int *__restrict__ qord, const float4 *__restrict__ spts,
+    const int *__restrict__ start, const GridParams *__restrict__ gp,
     int self_exclude, int k, float *__restrict__ od, int *__restrict__ oi) {
+  __shared__ int s_run[D == 3 ? 18 : 6][kSBlock];  // each thread its own column
   const int lane = blockIdx.x * kSBlock + threadIdx.x;
   if (lane >= nq) return;
   const int i = qord[lane];
@@ -629,14 +621,48 @@ __global__ __launch_bounds__(kSBlock) void k_knn_grid(
     // ring beyond which no cell is left
     int rall = max(max(cx, g.nx - 1 - cx), max(cy, g.ny - 1 - cy));
     if (D == 3) rall = max(rall, max(cz, g.nz - 1 - cz));
-    for (int r = 0;; ++r) {
+    // Rings 0 and 1: cells that follow each other along x hold consecutive
+    // candidates, so the block is 9 (2-D: 3) runs.  Their bounds are fetched
+    // together (LDS), and a lane goes through its runs without waiting for the
+    // others', the next candidate on its way while one is looked at.
+    constexpr int NR = D == 3 ? 9 : 3;
+    const int tid = threadIdx.x;
+    const int x0 = max(cx - 1, 0), x1 = min(cx + 1, g.nx - 1);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int y = cy - 1 + (D == 3 ? r % 3 : r), z = cz + (D == 3 ? r / 3 - 1 : 0);
+      const bool in = y >= 0 && y < g.ny && z >= 0 && z < g.nz;
+      const int row = in ? (z * g.ny + y) * g.nx : 0;
+      s_run[2 * r][tid] = in ? start[row + x0] : 0;
+      s_run[2 * r + 1][tid] = in ? start[row + x1 + 1] : 0;
+    }
+    int run = 0, p0 = s_run[0][tid], p1 = s_run[1][tid];
+    auto skip = [&]() {  // to the next run with a candidate; false: none is left
+      while (p0 >= p1 && ++run < NR) {
+        p0 = s_run[2 * run][tid];
+        p1 = s_run[2 * run + 1][tid];
+      }
+      return p0 < p1;
+    };
+    bool have = skip();
+    float4 next = spts[have ? p0 : 0];
+    while (have) {
+      const float4 p = next;
+      ++p0;
+      have = skip();
+      if (have) next = spts[p0];
+      grid_candidate<D, K>(q, i, self_exclude, p, bd, bi);
+    }
+    bool more = rall > 1 && !(bi[K - 1] >= 0 &&
+                              unvisited_dist2<D>(q, cx, cy, cz, 1, g) * (1.0 - 1e-4) > (double)bd[K - 1]);
+    for (int r = 2; more; ++r) {
       if (r > kRingFallback) {
 #pragma unroll
         for (int s = 0; s < K; ++s) {
           bd[s] = __builtin_huge_valf();
           bi[s] = -1;
         }
-        grid_visit<D, K>(q, i, self_exclude, 0, g.nvalid, spts, sidx, bd, bi);
+        grid_visit<D, K>(q, i, self_exclude, 0, g.nvalid, spts, bd, bi);
         break;
       }
       const int zr = D == 3 ? r : 0;
@@ -650,7 +676,7 @@ __global__ __launch_bounds__(kSBlock) void k_knn_grid(
           if (D == 2) {
             if (!edge) continue;
             const int cell = y * g.nx + x;
-            grid_visit<D, K>(q, i, self_exclude, start[cell], start[cell + 1], spts, sidx, bd, bi);
+            grid_visit<D, K>(q, i, self_exclude, start[cell], start[cell + 1], spts, bd, bi);
             continue;
           }
           // 3-D: the whole z column on the rim of the (a, b) square, else its two ends
@@ -659,7 +685,7 @@ __global__ __launch_bounds__(kSBlock) void k_knn_grid(
             const int z = cz + c;
             if (z < 0 || z >= g.nz) continue;
             const int cell = (z * g.ny + y) * g.nx + x;
-            grid_visit<D, K>(q, i, self_exclude, start[cell], start[cell + 1], spts, sidx, bd, bi);
+            grid_visit<D, K>(q, i, self_exclude, start[cell], start[cell + 1], spts, bd, bi);
           }
         }
       }
@@ -785,7 +811,7 @@ static int knn_grid(dugma_ctx *c, int D, int K, int k, const double *R, const do
                                              (int)(cap + 1), c->stream));
   const size_t need_m = R ? al((size_t)np * D * 4) : 0;
   const size_t b_part = al((size_t)kBoxGroups * 8 * 4), b_gp = al(sizeof(GridParams));
-  const size_t b_cnt = al((size_t)(cap + 1) * 4), b_pts = al((size_t)np * D * 4), b_idx = al((size_t)np * 4);
+  const size_t b_cnt = al((size_t)(cap + 1) * 4), b_pts = al((size_t)np * sizeof(float4)), b_idx = al((size_t)np * 4);
   const size_t b_tmp = al(temp_bytes), b_out = al((size_t)nq * k * 4), b_ord = al((size_t)nq * 4);
   int rc = c->scratch2.ensure(need_m + b_part + b_gp + 3 * b_cnt + b_pts + b_idx + b_tmp + 2 * b_out + b_ord);
   if (rc) return rc;
@@ -808,9 +834,9 @@ static int knn_grid(dugma_ctx *c, int D, int K, int k, const double *R, const do
   p += b_cnt;
   int *qord = (int *)p;
   p += b_ord;
-  float *spts = (float *)p;
+  float4 *spts = (float4 *)p;
   p += b_pts;
-  int *sidx = (int *)p;
+  int *sidx = self ? (int *)p : nullptr;  // the queries are the candidates: their order too
   p += b_idx;
   void *tmp = p;
   p += b_tmp;
@@ -836,20 +862,24 @@ static int knn_grid(dugma_ctx *c, int D, int K, int k, const double *R, const do
     hipLaunchKernelGGL(k_grid_scatter<3>, pgrid, blk, 0, c->stream, Pp, np, gp, start, cnt, spts, sidx);
   else
     hipLaunchKernelGGL(k_grid_scatter<2>, pgrid, blk, 0, c->stream, Pp, np, gp, start, cnt, spts, sidx);
-  // the candidate scatter has counted cnt back down to zero: reuse it
-  if (D == 3)
-    hipLaunchKernelGGL(k_query_count<3>, qgrid, blk, 0, c->stream, Qp, nq, gp, cnt);
-  else
-    hipLaunchKernelGGL(k_query_count<2>, qgrid, blk, 0, c->stream, Qp, nq, gp, cnt);
-  DUGMA_HIP(hipGetLastError());
-  DUGMA_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, temp_bytes, cnt, qstart, (int)(cap + 1), c->stream));
-  if (D == 3)
-    hipLaunchKernelGGL(k_query_scatter<3>, qgrid, blk, 0, c->stream, Qp, nq, gp, qstart, cnt, qord);
-  else
-    hipLaunchKernelGGL(k_query_scatter<2>, qgrid, blk, 0, c->stream, Qp, nq, gp, qstart, cnt, qord);
-  DUGMA_HIP(hipGetLastError());
+  if (!self) {
+    // the candidate scatter has counted cnt back down to zero: reuse it
+    if (D == 3)
+      hipLaunchKernelGGL(k_query_count<3>, qgrid, blk, 0, c->stream, Qp, nq, gp, cnt);
+    else
+      hipLaunchKernelGGL(k_query_count<2>, qgrid, blk, 0, c->stream, Qp, nq, gp, cnt);
+    DUGMA_HIP(hipGetLastError());
+    DUGMA_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, temp_bytes, cnt, qstart, (int)(cap + 1), c->stream));
+    if (D == 3)
+      hipLaunchKernelGGL(k_query_scatter<3>, qgrid, blk, 0, c->stream, Qp, nq, gp, qstart, cnt, qord);
+    else
+      hipLaunchKernelGGL(k_query_scatter<2>, qgrid, blk, 0, c->stream, Qp, nq, gp, qstart, cnt, qord);
+    DUGMA_HIP(hipGetLastError());
+  } else {
+    qord = sidx;
+  }
 #define KNN_GRID(DD, KK)                                                                               \
-  hipLaunchKernelGGL((k_knn_grid<DD, KK>), qgrid, blk, 0, c->stream, Qp, nq, qord, spts, sidx, start, gp, \
+  hipLaunchKernelGGL((k_knn_grid<DD, KK>), qgrid, blk, 0, c->stream, Qp, nq, qord, spts, start, gp, \
                      self, k, od, oi)
   if (D == 3) {
     if (K == 8) KNN_GRID(3, 8); else if (K == 16) KNN_GRID(3, 16); else KNN_GRID(3, 32);
