@@ -841,19 +841,22 @@ static int transform_sources(dugma_ctx *c, const PoseArg &ps, bool iso, float la
 }
 
 // Bound of R's largest singular value squared (1 for a rotation): what R can
-// do to a covariance's largest eigenvalue.
+// do to a covariance's largest eigenvalue.  Infinite (every pair counts) for an R
+// so far from a similarity that it also spoils a covariance's conditioning.
 static float pose_lam_scale(int D, const double *R) {
-  double big = 0.0;
+  double big = 0.0, small = INFINITY;
   for (int a = 0; a < D; ++a) {
-    double row = 0.0;
+    double row = 0.0, diag = 0.0;
     for (int b = 0; b < D; ++b) {
       double v = 0.0;
       for (int k = 0; k < D; ++k) v += R[k + D * a] * R[k + D * b];
       row += std::fabs(v);
+      if (a == b) diag = v;
     }
     big = std::max(big, row);
+    small = std::min(small, 2.0 * diag - row);
   }
-  return (float)(big * 1.000001);
+  return small > 0.25 * big ? (float)(big * 1.000001) : INFINITY;
 }
 
 static int resolve_iso(dugma_ctx *c, int cov_mode, bool *iso) {

@@ -7,7 +7,8 @@
 // d^T S^-1 d >= |d|^2 / (lam_p + lam_q), lam the largest eigenvalue of each
 // point's covariance, so every pair with |d|^2 > kZeroDist2 (lam_p + lam_q) is
 // such a pair.  kZeroDist2 = 126 * 2 ln 2 plus 1% for the rounding of the FP32
-// exponent.
+// exponent; lam itself is raised where a covariance's conditioning makes that
+// rounding larger.
 //
 // Each cloud's kept points are put once, at init, into the order of a Hilbert
 // curve; 64 consecutive ones are a block with a bounding box and the largest

@@ -67,26 +67,40 @@ __global__ __launch_bounds__(kNBlock) void k_near_keys(const float *__restrict__
   val[q] = q;
 }
 
+// How much a covariance's conditioning loosens the bound: the FP32 determinant
+// of a pair's S is off by up to 1e-6 of its mean eigenvalue cubed (in 2-D
+// squared), so d^T S^-1 d by that share of 1 / dn, dn the determinant over that
+// cube; by Minkowski's inequality a pair is no worse than three times its worse
+// point.  Near 1e-6 the FP32 determinant can come out as 0 or negative and the
+// term as a NaN: such a point counts as near everything.
+__device__ __forceinline__ float lam_slack(float dn) {
+  return dn > 4e-6f ? 1.001f + 6e-6f / dn : __builtin_huge_valf();
+}
 // Largest eigenvalue of a symmetric covariance (closed form, FP32), raised by
-// 1e-3 so that it is a bound.
+// 1e-3 and by lam_slack so that it is a bound.
 __device__ __forceinline__ float lam_max3(float s11, float s12, float s13, float s22, float s23, float s33) {
   const float m = (s11 + s22 + s33) * (1.0f / 3.0f);
   const float d1 = s11 - m, d2 = s22 - m, d3 = s33 - m;
   const float o2 = s12 * s12 + s13 * s13 + s23 * s23;
   const float p = sqrtf((d1 * d1 + d2 * d2 + d3 * d3 + 2.0f * o2) * (1.0f / 6.0f));
   if (!(p > 1e-6f * m)) return m * 1.001f + 2.0f * p;  // s I (or NaN)
+  const float im = 1.0f / m;
+  const float n11 = s11 * im, n22 = s22 * im, n33 = s33 * im, n12 = s12 * im, n13 = s13 * im, n23 = s23 * im;
+  const float dn = n11 * (n22 * n33 - n23 * n23) - n12 * (n12 * n33 - n23 * n13) + n13 * (n12 * n23 - n22 * n13);
   const float ip = 1.0f / p;
   const float b11 = d1 * ip, b22 = d2 * ip, b33 = d3 * ip, b12 = s12 * ip, b13 = s13 * ip, b23 = s23 * ip;
   const float det = b11 * (b22 * b33 - b23 * b23) - b12 * (b12 * b33 - b23 * b13) + b13 * (b12 * b23 - b22 * b13);
   const float r = fminf(1.0f, fmaxf(-1.0f, 0.5f * det));
-  return (m + 2.0f * p * cosf(acosf(r) * (1.0f / 3.0f))) * 1.001f;
+  return (m + 2.0f * p * cosf(acosf(r) * (1.0f / 3.0f))) * lam_slack(dn);
 }
 __device__ __forceinline__ float rec_lam(const Rec3F &r) {
   return lam_max3(r.s11, r.s12, r.s13, r.s22, r.s23, r.s33);
 }
 __device__ __forceinline__ float rec_lam(const Rec2F &r) {
   const float h = 0.5f * (r.s11 + r.s22), d = 0.5f * (r.s11 - r.s22);
-  return (h + sqrtf(d * d + r.s12 * r.s12)) * 1.001f;
+  const float ih = 1.0f / h;
+  const float dn = (r.s11 * ih) * (r.s22 * ih) - (r.s12 * ih) * (r.s12 * ih);
+  return (h + sqrtf(d * d + r.s12 * r.s12)) * lam_slack(dn);
 }
 __device__ __forceinline__ void rec_pos(const Rec3F &r, float *x) { x[0] = r.hx; x[1] = r.hy; x[2] = r.hz; }
 __device__ __forceinline__ void rec_pos(const Rec3I &r, float *x) { x[0] = r.hx; x[1] = r.hy; x[2] = r.hz; }
