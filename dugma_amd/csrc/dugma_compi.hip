@@ -56,8 +56,8 @@ struct CompiPose {
   float gsc;    // sqrtf(Isig^3) in 3-D (compi.cu:662), Isig in 2-D (compi.cu:126)
 };
 
-// Streamed target record: the exponent's inputs in FP64 (the quadratic
-// form of B = fl32(inv(CX) Isig) as [B11 B22 B33 2B12 2B13 2B23] (2-D
+// Streamed target record: the exponent's inputs in FP64 (-log2(e)/2 times the
+// quadratic form of B = fl32(inv(CX) Isig) as [B11 B22 B33 2B12 2B13 2B23] (2-D
 // [B11 B22 2B12]) and lg = log2(fl32(gX gsc))), then n, sym(B) and the
 // features n n^T, n^T B n, (B+B^T) n in FP32.  3-D 144 B, 2-D 80 B.
 struct alignas(16) TgtRec3 {
@@ -73,7 +73,7 @@ struct alignas(16) TgtRec2 {
 static_assert(sizeof(TgtRec3) == 144 && sizeof(TgtRec2) == 80, "target record layout");
 
 // Per-lane source record: C = R A^T R^T (2-D R A R^T) as a quadratic form
-// in FP64 ([C11 C22 C33 2C12 2C13 2C23]), m' = R y + t as FP32 hi + lo, and
+// in FP64, times -log2(e)/2 ([C11 C22 C33 2C12 2C13 2C23]), m' = R y + t as FP32 hi + lo, and
 // gY fl32(gsc).  3-D 80 B, 2-D 48 B.
 struct alignas(16) SrcRec3 {
   double q[6];
@@ -134,6 +134,7 @@ __device__ void compi_tgt(int i, const float *__restrict__ X, const float *__res
     r.q[3] = (double)B[3] + (double)B[1];
     r.q[4] = (double)B[6] + (double)B[2];
     r.q[5] = (double)B[7] + (double)B[5];
+    for (double &q : r.q) q *= kNegHalfLog2eD;
     r.lg = lg;
     r.s = (float)s;
     reinterpret_cast<TgtRec3 *>(outv)[i] = r;
@@ -151,6 +152,7 @@ __device__ void compi_tgt(int i, const float *__restrict__ X, const float *__res
     r.q[0] = B[0];
     r.q[1] = B[3];
     r.q[2] = (double)B[2] + (double)B[1];
+    for (double &q : r.q) q *= kNegHalfLog2eD;
     r.lg = lg;
     r.s = (float)s;
     reinterpret_cast<TgtRec2 *>(outv)[i] = r;
@@ -210,6 +212,7 @@ __device__ void compi_src(int j, const float *__restrict__ Y, const float *__res
     r.q[3] = C[3] + C[1];
     r.q[4] = C[6] + C[2];
     r.q[5] = C[7] + C[5];
+    for (double &q : r.q) q *= kNegHalfLog2eD;
     for (int a = 0; a < 3; ++a) {
       r.mh[a] = mh[a];
       r.ml[a] = ml[a];
@@ -222,6 +225,7 @@ __device__ void compi_src(int j, const float *__restrict__ Y, const float *__res
     r.q[0] = C[0];
     r.q[1] = C[3];
     r.q[2] = C[2] + C[1];
+    for (double &q : r.q) q *= kNegHalfLog2eD;
     for (int a = 0; a < 2; ++a) {
       r.mh[a] = mh[a];
       r.ml[a] = ml[a];
@@ -248,7 +252,10 @@ __global__ __launch_bounds__(kCBlock) void k_compi_prep(
 
 // W_j = sum_i P_ij G_i.  Lane = source j (stationary, 64 per workgroup); the
 // workgroup's target chunk is split into kCWaves contiguous parts, one per
-// wave, streamed through SGPRs one record ahead (index clamped to the part).
+// wave; the exponents' inputs are streamed through SGPRs one record ahead (index
+// clamped to the part), the features of a sub-tile lie in LDS (an FMA with an
+// SGPR operand issues in 4.5 cycles, with VGPRs only in 2.5).  Bound by VALU
+// issue: 6,000 x 6,000 in 103 us, 114 with the features in SGPRs too.
 // Per pair: d = n_i - m'_j in FP64, e1 = -log2(e)/2 d^T C_j d + lg_i,
 // e2 = -log2(e)/2 d^T B_i d + lg_i (FP64), P 2^-o = exp2(e1 - o) + exp2(e2 - o)
 // in FP32 with the lane's running scale o.  The sums are FP32 over sub-tiles
@@ -256,12 +263,20 @@ __global__ __launch_bounds__(kCBlock) void k_compi_prep(
 // 2^o in FP64 and the waves' sums meet in LDS in a fixed order:
 // (w0 + w2) + (w1 + w3).
 template <int D>
-__global__ __launch_bounds__(kCBlock) void k_compi_w(
+__global__ __launch_bounds__(kCBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_compi_w(
     const void *__restrict__ srcv, int M, const void *__restrict__ tgtv, int N,
     int chunk, double *__restrict__ part) {
-  constexpr int NW = D == 3 ? 20 : 12;
+  constexpr int NW = D == 3 ? 20 : 12, NS = D == 3 ? 6 : 3;
   using Tgt = typename std::conditional<D == 3, TgtRec3, TgtRec2>::type;
   using Src = typename std::conditional<D == 3, SrcRec3, SrcRec2>::type;
+  struct Exp {  // a record's part that is streamed through SGPRs: the exponents' inputs
+    double q[NS], lg;
+    float n[D];
+    __device__ __forceinline__ explicit Exp(const Tgt &t) : lg(t.lg) {
+      for (int a = 0; a < NS; ++a) q[a] = t.q[a];
+      for (int a = 0; a < D; ++a) n[a] = t.n[a];
+    }
+  };
   const Tgt *__restrict__ T = reinterpret_cast<const Tgt *>(tgtv);
   // the wave index is uniform: say so, so the target stream uses scalar loads
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -281,36 +296,53 @@ __global__ __launch_bounds__(kCBlock) void k_compi_w(
   double W[NW];
 #pragma unroll
   for (int k = 0; k < NW; ++k) W[k] = 0.0;
-  double o = -INFINITY;  // running scale (log2) of this lane's sums
+  double o = -INFINITY, orise = -INFINITY;  // running scale (log2) of this lane's sums; what raises it
+  constexpr int F = NW - 1, F4 = (F + 3) / 4;  // features of a target
+  union Shared {
+    float4 feat[kCWaves][F4][kCSub];  // a sub-tile's features, per wave
+    double red[2][NW][64];
+  };
+  __shared__ Shared sh;
+  float4(*feat)[kCSub] = sh.feat[wave];
   if (i0 < i1) {
-    Tgt tn = T[i0];
+    Exp tn(T[i0]);
     for (int s0 = i0; s0 < i1; s0 += kCSub) {
       float w[NW];
 #pragma unroll
       for (int k = 0; k < NW; ++k) w[k] = 0.0f;
       const int s1 = min(s0 + kCSub, i1);
+      {
+        // in the order of w[1 ..]: n, n n^T, n^T B n, (B+B^T) n, sym(B)
+        const Tgt t = T[min(s0 + lane, s1 - 1)];
+        float f[4 * F4] = {};
+        int q = 0;
+        for (int a = 0; a < D; ++a) f[q++] = t.n[a];
+        for (int a = 0; a < NS; ++a) f[q++] = t.nn[a];
+        f[q++] = t.s;
+        for (int a = 0; a < D; ++a) f[q++] = t.v[a];
+        for (int a = 0; a < NS; ++a) f[q++] = t.b[a];
+#pragma unroll
+        for (int a = 0; a < F4; ++a) feat[a][lane] = make_float4(f[4 * a], f[4 * a + 1], f[4 * a + 2], f[4 * a + 3]);
+      }
+      wave_lds_fence();
       for (int i = s0; i < s1; ++i) {
-        const Tgt t = tn;
-        tn = T[min(i + 1, i1 - 1)];
+        const Exp t = tn;
+        tn = Exp(T[min(i + 1, i1 - 1)]);
         double e1, e2;
         if constexpr (D == 3) {
           const double dx = (double)t.n[0] - m[0], dy = (double)t.n[1] - m[1], dz = (double)t.n[2] - m[2];
           const double xx = dx * dx, yy = dy * dy, zz = dz * dz, xy = dx * dy, xz = dx * dz, yz = dy * dz;
-          const double mal1 = fma(cq[0], xx, fma(cq[1], yy, fma(cq[2], zz, fma(cq[3], xy, fma(cq[4], xz, cq[5] * yz)))));
-          const double mal2 =
-              fma(t.q[0], xx, fma(t.q[1], yy, fma(t.q[2], zz, fma(t.q[3], xy, fma(t.q[4], xz, t.q[5] * yz)))));
-          e1 = fma(mal1, kNegHalfLog2eD, t.lg);
-          e2 = fma(mal2, kNegHalfLog2eD, t.lg);
+          e1 = fma(cq[0], xx, fma(cq[1], yy, fma(cq[2], zz, fma(cq[3], xy, fma(cq[4], xz, fma(cq[5], yz, t.lg))))));
+          e2 = fma(t.q[0], xx,
+                   fma(t.q[1], yy, fma(t.q[2], zz, fma(t.q[3], xy, fma(t.q[4], xz, fma(t.q[5], yz, t.lg))))));
         } else {
           const double dx = (double)t.n[0] - m[0], dy = (double)t.n[1] - m[1];
           const double xx = dx * dx, yy = dy * dy, xy = dx * dy;
-          const double mal1 = fma(cq[0], xx, fma(cq[1], yy, cq[2] * xy));
-          const double mal2 = fma(t.q[0], xx, fma(t.q[1], yy, t.q[2] * xy));
-          e1 = fma(mal1, kNegHalfLog2eD, t.lg);
-          e2 = fma(mal2, kNegHalfLog2eD, t.lg);
+          e1 = fma(cq[0], xx, fma(cq[1], yy, fma(cq[2], xy, t.lg)));
+          e2 = fma(t.q[0], xx, fma(t.q[1], yy, fma(t.q[2], xy, t.lg)));
         }
         const double em = fmax(e1, e2);
-        if (em > o + kRescale) {
+        if (em > orise) {
           // the lane's largest weight so far: rescale its sums (rare)
           const float f = __builtin_amdgcn_exp2f((float)(o - em));
 #pragma unroll
@@ -319,32 +351,23 @@ __global__ __launch_bounds__(kCBlock) void k_compi_w(
             W[k] *= (double)f;
           }
           o = em;
+          orise = em + kRescale;
         }
         const float P = __builtin_amdgcn_exp2f((float)(e1 - o)) + __builtin_amdgcn_exp2f((float)(e2 - o));
-        if constexpr (D == 3) {
-          w[0] += P;
+        w[0] += P;
+        float f[4 * F4];
 #pragma unroll
-          for (int a = 0; a < 3; ++a) w[1 + a] = fmaf(P, t.n[a], w[1 + a]);
-#pragma unroll
-          for (int a = 0; a < 6; ++a) w[4 + a] = fmaf(P, t.nn[a], w[4 + a]);
-          w[10] = fmaf(P, t.s, w[10]);
-#pragma unroll
-          for (int a = 0; a < 3; ++a) w[11 + a] = fmaf(P, t.v[a], w[11 + a]);
-#pragma unroll
-          for (int a = 0; a < 6; ++a) w[14 + a] = fmaf(P, t.b[a], w[14 + a]);
-        } else {
-          w[0] += P;
-#pragma unroll
-          for (int a = 0; a < 2; ++a) w[1 + a] = fmaf(P, t.n[a], w[1 + a]);
-#pragma unroll
-          for (int a = 0; a < 3; ++a) w[3 + a] = fmaf(P, t.nn[a], w[3 + a]);
-          w[6] = fmaf(P, t.s, w[6]);
-#pragma unroll
-          for (int a = 0; a < 2; ++a) w[7 + a] = fmaf(P, t.v[a], w[7 + a]);
-#pragma unroll
-          for (int a = 0; a < 3; ++a) w[9 + a] = fmaf(P, t.b[a], w[9 + a]);
+        for (int a = 0; a < F4; ++a) {
+          const float4 u = feat[a][i - s0];
+          f[4 * a] = u.x;
+          f[4 * a + 1] = u.y;
+          f[4 * a + 2] = u.z;
+          f[4 * a + 3] = u.w;
         }
+#pragma unroll
+        for (int k = 0; k < F; ++k) w[1 + k] = fmaf(P, f[k], w[1 + k]);
       }
+      wave_lds_fence();
 #pragma unroll
       for (int k = 0; k < NW; ++k) W[k] += (double)w[k];
     }
@@ -353,7 +376,8 @@ __global__ __launch_bounds__(kCBlock) void k_compi_w(
   const double sc = o == -INFINITY ? 0.0 : exp2(o);
 #pragma unroll
   for (int k = 0; k < NW; ++k) W[k] *= sc;
-  __shared__ double red[2][NW][64];
+  double(&red)[2][NW][64] = sh.red;
+  __syncthreads();  // the features have been read
   if (wave >= 2)
 #pragma unroll
     for (int k = 0; k < NW; ++k) red[wave - 2][k][lane] = W[k];
