@@ -829,7 +829,8 @@ def main():
                      "traffic": PROFILED_TRAFFIC_200K_ISO if fused["plan"] == TRAFFIC_PLAN else None,
                      "traffic_source": TRAFFIC_PROFILE,
                      "kernel_ms": round(fused["kernel_ms"], 4), "flop_per_pair": FLOP_3D_ISO_FUSED,
-                     "launch": fused["plan"]},
+                     "pairs": "all of the sum; those whose FP32 term is exactly zero are found and not "
+                              "evaluated, so frac can exceed 1", "launch": fused["plan"]},
         "init_ms": round(fused["init_ms"], 3),
     }
     if only == "fused":

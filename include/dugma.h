@@ -297,7 +297,7 @@ typedef struct {
   int use_graph;             /* replay one captured iteration (hipGraph) */
   int one_trial_per_launch;  /* baseline: trials one after another, host check per step */
   int check_every;           /* graph mode: host checks for completion every n steps */
-  int grid;                  /* workgroups of the persistent pair kernel (0: from the launch shape) */
+  int grid;                  /* workgroups of the pair kernel (0: from the launch shape) */
   int sigma_update;          /* 1: DUGMA sigma update (one extra measuring pass first) */
   double relax;              /* > 1: over-relax the pose step once annealing has ended
                                 (rotation angle and centroid move times relax) */
@@ -351,10 +351,11 @@ int dugma_batch_register(dugma_batch *b, const double *R0, const double *t0,
                          int *iters, int *status, double *E);
 int dugma_batch_info(const dugma_batch *b, int *ntrials, int *nitems,
                      long long *pairs_per_iteration);
-/* Launch shape of the persistent pair kernels: waves per workgroup (1, 2, 4;
- * the target tile is 64 x waves points) and source chunks per target tile
- * for each of 4 size classes of trials (source count < 1000, < 2000, < 4000,
- * more), and resident waves, per level (0: full clouds, 1: every 4th point).
+/* Launch shape of the pair kernels: units of 64 targets per target tile
+ * (waves: 1, 2, 4; the tile is 64 x waves points) and source chunks per target
+ * tile for each of 4 size classes of trials (source count < 1000, < 2000, < 4000,
+ * more), and resident waves (beyond 64 times them the launch is persistent),
+ * per level (0: full clouds, 1: every 4th point).
  * dugma_batch_autotune times whole isotropic iterations -- plus, once
  * dugma_batch_set_covariances has run, whole refinement passes, their sum
  * being the figure minimised -- from the poses R0, t0 on the batch's own

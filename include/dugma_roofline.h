@@ -1,6 +1,8 @@
 /* dugma_roofline.h -- canonical algorithmic FLOP per point pair of the pair
  * kernels, the numerator of every roofline figure reported for this library
- * (achieved FLOP/s = pairs per second x FLOP per pair).
+ * (achieved FLOP/s = pairs per second x FLOP per pair).  All pairs of a sum
+ * count, also those that the energy passes leave out because their FP32 term
+ * is exactly zero; such a figure can exceed the peak.
  *
  * Counting: an FMA is 2 FLOP; each exp, rsq and rcp is 1.  The per-source
  * preparation (R x_j + t and R S_j R^T) is O(M) and not counted.
