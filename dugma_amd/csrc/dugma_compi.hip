@@ -22,7 +22,7 @@
 //     least 2^16), so that exp2 runs in FP32 on arguments <= 16 and pairs far
 //     below FP32's range keep their FP64 weight; the scale is applied to the
 //     lane's FP64 sums at the end.
-//  2. k_compi_mom: per block of 32 sources, the chunk partials are summed
+//  2. k_compi_mom: per block of 8 (or 32) sources, the chunk partials are summed
 //     into the features, staged in LDS, and the 325 (85) moments
 //     sum_j W'_j,f * m'_j.. * A'_j,.. accumulated; k_compi_msum adds the
 //     block partials, one wave per moment.
@@ -44,7 +44,11 @@ namespace dugma {
 constexpr int kCBlock = 256;
 constexpr int kCWaves = kCBlock / 64;  // waves per workgroup of k_compi_w
 constexpr int kCSub = 64;
-constexpr int kMomSrc = 32;            // sources per workgroup of k_compi_mom
+// Sources per workgroup of k_compi_mom: few, so that the sums over the chunk
+// partials are one load per thread deep (6,000 sources: 9 us, with 32 a workgroup
+// 20.6), more where the workgroups fill the chip anyway and their partials (325
+// doubles each) would only take memory.
+constexpr int kMomSrc = 8, kMomSrcMany = 32, kMomMany = 65536;
 constexpr int kFeat = 32;  // per-source feature stride (doubles) for the moments
 constexpr double kNegHalfLog2eD = -0.72134752044448170368;  // -log2(e) / 2
 constexpr double kRescale = 16.0;  // a lane's scale rises when an exponent exceeds it by this (log2)
@@ -398,7 +402,7 @@ __global__ __launch_bounds__(kCBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 }
 
 // Moments: mom[k] = sum_j prod of up to four feature entries of source j
-// (index -1 = 1).  One workgroup per kMomSrc sources: their features (the W
+// (index -1 = 1).  One workgroup per MS sources: their features (the W
 // partials summed over the target chunks in a fixed order, times gY_j, plus
 // m' and A' from k_compi_prep) are staged in LDS, then each thread
 // accumulates its moments over them.  Block partials are summed later.
@@ -406,7 +410,7 @@ struct MomTab {
   short ix[400][4];
 };
 
-template <int D>
+template <int D, int MS>
 __global__ __launch_bounds__(kCBlock) void k_compi_mom(
     const double *__restrict__ wpart, int M, int nchunks,
     const void *__restrict__ srcv, const double *__restrict__ feat, int nmom,
@@ -414,9 +418,9 @@ __global__ __launch_bounds__(kCBlock) void k_compi_mom(
   constexpr int NW = D == 3 ? 20 : 12;
   using Src = typename std::conditional<D == 3, SrcRec3, SrcRec2>::type;
   const Src *__restrict__ src = reinterpret_cast<const Src *>(srcv);
-  __shared__ double fs[kMomSrc][kFeat];
-  const int j0 = blockIdx.x * kMomSrc;
-  for (int e = threadIdx.x; e < kMomSrc * kFeat; e += kCBlock) {
+  __shared__ double fs[MS][kFeat];
+  const int j0 = blockIdx.x * MS;
+  for (int e = threadIdx.x; e < MS * kFeat; e += kCBlock) {
     const int jl = e / kFeat, k = e % kFeat, j = j0 + jl;
     double v = 0.0;
     if (j < M) {
@@ -446,7 +450,7 @@ __global__ __launch_bounds__(kCBlock) void k_compi_mom(
   for (int k = threadIdx.x; k < nmom; k += kCBlock) {
     const int a = tab.ix[k][0], b = tab.ix[k][1], c = tab.ix[k][2], d = tab.ix[k][3];
     double s = 0.0;
-    for (int jl = 0; jl < kMomSrc; ++jl) {
+    for (int jl = 0; jl < MS; ++jl) {
       double v = fs[jl][a];
       if (b >= 0) v *= fs[jl][b];
       if (c >= 0) v *= fs[jl][c];
@@ -770,7 +774,8 @@ extern "C" int dugma_compi(dugma_ctx *ctx, const double *R, const double *t,
   nch = std::max(1, std::min(nch, std::max(1, n / (kCWaves * 64))));
   const int chunk = (n + nch - 1) / nch;
   const int nchunks = (n + chunk - 1) / chunk;
-  const int mblocks = (m + kMomSrc - 1) / kMomSrc;
+  const bool many = m > kMomMany;
+  const int mblocks = many ? (m + kMomSrcMany - 1) / kMomSrcMany : (m + kMomSrc - 1) / kMomSrc;
   // scratch: tgt records | src | feat | W partials | moment partials | moments
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t o_src = al(trec * n);
@@ -798,12 +803,22 @@ extern "C" int dugma_compi(dugma_ctx *ctx, const double *R, const double *t,
     hipLaunchKernelGGL(k_compi_prep<3>, dim3(pgrid), blk, 0, c->stream, c->dX, c->dXCinv, c->dgX, n, c->dY,
                        c->dYCinv, c->dgY, m, ps, tgt, src, feat);
     hipLaunchKernelGGL(k_compi_w<3>, dim3(sblocks, nchunks), blk, 0, c->stream, src, m, tgt, n, chunk, wpart);
-    hipLaunchKernelGGL(k_compi_mom<3>, dim3(mblocks), blk, 0, c->stream, wpart, m, nchunks, src, feat, nmom, tab, mpart);
+    if (many)
+      hipLaunchKernelGGL((k_compi_mom<3, kMomSrcMany>), dim3(mblocks), blk, 0, c->stream, wpart, m, nchunks, src, feat,
+                         nmom, tab, mpart);
+    else
+      hipLaunchKernelGGL((k_compi_mom<3, kMomSrc>), dim3(mblocks), blk, 0, c->stream, wpart, m, nchunks, src, feat,
+                         nmom, tab, mpart);
   } else {
     hipLaunchKernelGGL(k_compi_prep<2>, dim3(pgrid), blk, 0, c->stream, c->dX, c->dXCinv, c->dgX, n, c->dY,
                        c->dYCinv, c->dgY, m, ps, tgt, src, feat);
     hipLaunchKernelGGL(k_compi_w<2>, dim3(sblocks, nchunks), blk, 0, c->stream, src, m, tgt, n, chunk, wpart);
-    hipLaunchKernelGGL(k_compi_mom<2>, dim3(mblocks), blk, 0, c->stream, wpart, m, nchunks, src, feat, nmom, tab, mpart);
+    if (many)
+      hipLaunchKernelGGL((k_compi_mom<2, kMomSrcMany>), dim3(mblocks), blk, 0, c->stream, wpart, m, nchunks, src, feat,
+                         nmom, tab, mpart);
+    else
+      hipLaunchKernelGGL((k_compi_mom<2, kMomSrc>), dim3(mblocks), blk, 0, c->stream, wpart, m, nchunks, src, feat,
+                         nmom, tab, mpart);
   }
   // moment sums straight into the context's pinned result slots
   double *slots = c->hres + dugma_ctx::kResMoments;
